@@ -140,57 +140,17 @@ __device__ __forceinline__ float wave_max_xor_16_32(float x) {
     return rows_reduce(x, MaxOp{});
 }
 
+// A value every lane of the wave holds, in scalar registers.
+__device__ __forceinline__ unsigned long long uniform64(unsigned long long x) {
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(x));
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(x >> 32));
+    return (static_cast<unsigned long long>(hi) << 32) | lo;
+}
+
 // Raw v_exp_f32: no denormal range fix-up (results below 2^-126 flush to 0, which
 // only drops probabilities that are already negligible); exp2(-inf) == 0.
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-
-// Packed work items of a batch: sequence b owns ceil(L_b / split tokens) * kv_heads
-// items (none past *count_ptr).  Every workgroup scans the per-sequence counts
-// (256 sequences per pass, Hillis-Steele in LDS) and finds the item at index
-// `id`; false if the batch holds fewer items.  Called by every thread of the
-// workgroup (barriers inside); the first 256 threads do the scan.
-__device__ bool locate_item(const SplitArgs& a, uint32_t cpw, uint32_t id, uint32_t& b_out, uint32_t& h_out,
-                            uint32_t& split_out) {
-    __shared__ uint32_t s_scan[256];
-    __shared__ uint32_t s_hit[3];
-    const uint32_t tid = threadIdx.x;
-    const uint32_t tps = kWavesPerWg * cpw * kChunk;
-    const uint32_t H = a.g.kv_heads;
-    const uint32_t count = a.count_ptr ? min(a.batch, *a.count_ptr) : a.batch;
-    if (tid == 0) s_hit[0] = 0xffffffffu;
-    uint32_t base = 0;
-    const bool scans = tid < 256;
-    for (uint32_t b0 = 0; b0 < count; b0 += 256) {
-        const uint32_t bb = b0 + tid;
-        const uint32_t nsplit = scans && bb < count ? (split_length(a, bb) + tps - 1) / tps : 0;
-        const uint32_t n = nsplit * H;
-        if (scans) s_scan[tid] = n;
-        __syncthreads();
-        for (uint32_t off = 1; off < 256; off <<= 1) {
-            const uint32_t add = scans && tid >= off ? s_scan[tid - off] : 0;
-            __syncthreads();
-            if (scans) s_scan[tid] += add;
-            __syncthreads();
-        }
-        const uint32_t incl = base + (scans ? s_scan[tid] : 0);
-        const uint32_t excl = incl - n;
-        if (scans && id >= excl && id < incl) {
-            const uint32_t rem = id - excl;
-            s_hit[0] = bb;
-            s_hit[1] = rem / nsplit;
-            s_hit[2] = rem % nsplit;
-        }
-        base += s_scan[255];
-        __syncthreads();
-    }
-    __syncthreads();
-    if (s_hit[0] == 0xffffffffu) return false;
-    b_out = s_hit[0];
-    h_out = s_hit[1];
-    split_out = s_hit[2];
-    return true;
-}
 
 // The reference's K prologue for one row held one value per thread (thread t < D owns
 // dim t), in its own shape (qwen35_decoupled_k_norm_rope_kv_store_batch_quant_kernel,
@@ -246,7 +206,7 @@ __device__ void k_prologue(float& kx, float w, uint32_t tid, uint32_t position, 
 // every head) at slot nsplit, after the splits, which cover the L-1 cached keys.
 // The row and query loads go out before the context length arrives.
 template <uint32_t D>
-__device__ void append_record(const SplitArgs& a, uint32_t b, uint32_t h, uint32_t cpw) {
+__device__ void append_record(const SplitArgs& a, uint32_t b, uint32_t h) {
     constexpr uint32_t DJ = D / 64;
     __shared__ float s_k[D];
     __shared__ float s_v[D];
@@ -312,7 +272,10 @@ __device__ void append_record(const SplitArgs& a, uint32_t b, uint32_t h, uint32
     }
     __syncthreads();
     const uint32_t rec = record_floats(G, D);
-    float* r = a.part + ((static_cast<size_t>(b) * a.g.kv_heads + h) * (a.max_splits + 1) + split_count(L, cpw)) * rec;
+    const size_t bh = static_cast<size_t>(b) * a.g.kv_heads + h;
+    const size_t slot = a.stream_wgs != 0 ? static_cast<size_t>(a.batch) * a.g.kv_heads * a.max_splits + bh
+                                          : bh * (a.max_splits + 1) + split_count(L, a.cpw);
+    float* r = a.part + slot * rec;
     for (uint32_t i4 = tid; i4 < G * D / 4; i4 += 256) {
         const uint32_t d = (4 * i4) % D;
         *reinterpret_cast<float4*>(r + 4 * i4) = make_float4(s_v[d], s_v[d + 1], s_v[d + 2], s_v[d + 3]);
@@ -349,7 +312,7 @@ constexpr uint32_t decode_waves_per_eu() {
 // hold.  Otherwise (G > 8) the lo parts are a second fragment set and a second MFMA per
 // block.
 template <uint32_t D, bool QF32, bool APPEND, bool KF16 = false, bool VF16 = false, bool QPAIR = false,
-          bool CACHED = false>
+          bool CACHED = false, bool STREAM = false>
 __global__ void __launch_bounds__(64 * kWavesPerWg)
 __attribute__((amdgpu_waves_per_eu(decode_waves_per_eu<D, QF32 && !QPAIR, KF16, VF16>())))
 decode_kernel(SplitArgs a) {
@@ -365,13 +328,6 @@ decode_kernel(SplitArgs a) {
     static_assert(!APPEND || (!KF16 && !VF16), "the fused append stores q8 rows");
     extern __shared__ float smem[];
 
-    // Work item of this workgroup: one (sequence b, kv head h, split) of 4 waves x
-    // cpw steps.  One sequence: workgroup x = h * max_splits + split.  A batch: the
-    // items that hold keys are packed to the front of the grid (sequence-major,
-    // then head, then split), so whatever the lengths, the busy workgroups are the
-    // first ones dispatched and spread evenly over the XCDs and CUs; the grid's
-    // tail (bounded by max_context) exits at once.
-    const uint32_t cpw = launch_cpw(a);
     // Fused append: the last batch * kv_heads workgroups of the grid each handle the
     // new token of one (sequence, kv head).  Dispatched last, they take CU slots left
     // free by a small grid or freed by the first split workgroups to finish, so they
@@ -381,52 +337,14 @@ decode_kernel(SplitArgs a) {
         if (blockIdx.x >= first) {
             const uint32_t x = blockIdx.x - first;
             const uint32_t ab = x / a.g.kv_heads;
-            if (a.count_ptr == nullptr || ab < *a.count_ptr) append_record<D>(a, ab, x % a.g.kv_heads, cpw);
+            if (a.count_ptr == nullptr || ab < *a.count_ptr) append_record<D>(a, ab, x % a.g.kv_heads);
             return;
         }
     }
-    uint32_t split, h, b;
-    if (a.rowset_order) {
-        // Row sets of one sequence: items (kv head, split, row set), row sets fastest,
-        // each XCD (workgroup i runs on XCD i % 8) a contiguous range of them, so the
-        // workgroups an XCD runs together read the same keys (through its L2).  The
-        // grid is padded to a multiple of 8; items past a row set's splits exit.
-        const uint32_t total = a.max_splits * a.g.kv_heads * a.batch;
-        const uint32_t k = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
-        if (k >= total) return;
-        b = k % a.batch;
-        split = (k / a.batch) % a.max_splits;
-        h = k / a.batch / a.max_splits;
-        if (a.count_ptr != nullptr && b >= *a.count_ptr) return;
-    } else if (a.batch == 1) {
-        b = 0;
-        h = blockIdx.x / a.max_splits;
-        split = blockIdx.x % a.max_splits;
-    } else if (!locate_item(a, cpw, blockIdx.x, b, h, split)) {
-        return;
-    }
-    const uint32_t tid = threadIdx.x;
-    const uint32_t wave = tid >> 6;
-    const uint32_t lane = tid & 63;
-    const uint32_t g4 = lane >> 4;
-    const uint32_t n = lane & 15;
+    const uint32_t wave = STREAM ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
     const uint32_t G = a.group;
     const Geo& geo = a.g;
 
-    // Steps this wave may own, from the host bound alone: the first loads are issued
-    // before the context length arrives from memory.
-    // A split is 4*cpw consecutive steps.  At cpw == kInterleaveCpw wave w takes
-    // steps w, w+4, ... of it (the four waves of a workgroup then read one contiguous
-    // region at a time); otherwise each wave streams the w-th run of cpw steps.  A
-    // measured choice, not a model: config 2 shape, interleaved against runs, cpw 2
-    // (16k) +0.3 us, cpw 4 (32k) -0.4 us, cpw 8 (64k) +0.15 us.  The wave's local
-    // step i (0 <= i < n_steps) is split step first + i * stride.
-    const uint32_t nsteps_max = (a.max_context + kChunk - 1) / kChunk;
-    const bool interleave = cpw == kInterleaveCpw;
-    const uint32_t stride = interleave ? kWavesPerWg : 1u;
-    const uint32_t first = interleave ? split * kWavesPerWg * cpw + wave : (split * kWavesPerWg + wave) * cpw;
-    const uint32_t last_excl = min(interleave ? (split + 1) * kWavesPerWg * cpw : first + cpw, nsteps_max);
-    const uint32_t n_max = first < last_excl ? (last_excl - first + stride - 1) / stride : 0;
     const size_t slab_bytes = static_cast<size_t>(geo.page_tokens) * D;
 
     // Registers of one 32-token step: two K tiles, one V group, their scales.
@@ -436,6 +354,20 @@ decode_kernel(SplitArgs a) {
         ScaleVec ks, vs;
     };
 
+    // One run of steps of (sequence b, kv head h) by the four waves: this wave's local step
+    // i (0 <= i < n_max) is step first + i * stride of the sequence.  `split` is the run's
+    // number where the sequence is cut by itself (a run past the sequence's splits ends
+    // at once), 0 in a streamed plan; `mine` is the run's record.
+    auto run_steps = [&](uint32_t b, uint32_t h, uint32_t split, uint32_t first, uint32_t stride, uint32_t n_max,
+                         float* mine) __attribute__((always_inline)) {
+    // Streamed plan: the lane's position is made anew for each segment, so that the
+    // addresses derived from it are not kept in registers across the loop over segments
+    // (32 of D = 256's 256 registers went to scratch memory).
+    uint32_t tid = threadIdx.x;
+    if constexpr (STREAM) asm volatile("" : "+v"(tid));
+    const uint32_t lane = tid & 63;
+    const uint32_t g4 = lane >> 4;
+    const uint32_t n = lane & 15;
     // Load cursor: the page (slab) is looked up once per page, not per step.  Page
     // indices are clamped into the pool, so a speculative load past the sequence end
     // reads a valid (unused) page rather than whatever an unset table entry holds.
@@ -504,9 +436,8 @@ decode_kernel(SplitArgs a) {
         }
     }
     const uint32_t L = split_length(a, b);
-    const uint32_t tps = kWavesPerWg * cpw * kChunk;
-    const uint32_t nsplit = (L + tps - 1) / tps;
-    if (split >= nsplit) return;  // includes L == 0 (the combine kernel writes zeros)
+    // includes L == 0 (the combine kernel writes zeros)
+    if (!STREAM && split >= split_count(L, a.cpw)) return;
 
     // ---- Q fragments (B operand of the QK MFMA): lane (g4, n) holds head n,
     // dims 32*blk + 8*g4 .. +7 of every block.  Codes enter the MFMA as fp16
@@ -783,10 +714,8 @@ decode_kernel(SplitArgs a) {
     }
     __syncthreads();
 
-    // Partial record of one split: [O: G*D][m: G][l: G] padded to a multiple of 4 floats,
+    // Partial record of one run: [O: G*D][m: G][l: G] padded to a multiple of 4 floats,
     // so every record starts 16-byte aligned.
-    const uint32_t rec = record_floats(G, D);
-    float* mine = a.part + ((static_cast<size_t>(b) * geo.kv_heads + h) * (a.max_splits + 1) + split) * rec;
     for (uint32_t c4 = tid; c4 < G * D / 4; c4 += blockDim.x) {
         const uint32_t hn = (4 * c4) / D, dim = (4 * c4) % D;
         const uint32_t mt = dim / 16, gq = (dim % 16) / 4;
@@ -816,6 +745,105 @@ decode_kernel(SplitArgs a) {
             mine[G * D + G + hn] = Ls;
         }
     }
+    };
+
+    // The four waves take a run's steps interleaved at kInterleaveCpw steps per wave (the
+    // waves of a workgroup then read one contiguous region at a time), otherwise each
+    // wave streams its own consecutive steps.  A measured choice, not a model: config 2
+    // shape, interleaved against consecutive, cpw 2 (16k) +0.3 us, cpw 4 (32k) -0.4 us,
+    // cpw 8 (64k) +0.15 us.
+    const uint32_t rec = record_floats(G, D);
+    if constexpr (STREAM) {
+        // The segments of this workgroup's run (see StreamTotal).  What the loop carries is
+        // wave-uniform and kept in scalar registers; the lanes' sequences go to LDS (the
+        // wave's own part, so no barrier).
+        __shared__ unsigned long long s_before[kWavesPerWg][64];
+        __shared__ uint32_t s_steps[kWavesPerWg][64];
+        constexpr uint32_t kNew = APPEND ? 1u : 0u;
+        const uint32_t lane = threadIdx.x & 63;
+        const uint32_t H = geo.kv_heads;
+        unsigned long long at, end;
+        {
+            const StreamTotal total = stream_total(a, kNew);
+            const unsigned long long all = total.units * H;
+            at = uniform64(blockIdx.x * total.quota);
+            end = uniform64(min(all, at + total.quota));
+        }
+        uint32_t b0 = 0;
+        unsigned long long base = 0;
+        auto chunk = [&]() __attribute__((always_inline)) {
+            const StreamSeq q = stream_chunk(a, b0, base, kNew);
+            s_before[wave][lane] = q.before;
+            s_steps[wave][lane] = q.steps;
+        };
+        if (at < end) chunk();
+        while (at < end) {
+            // the lane whose sequence holds unit `at`
+            unsigned long long hit;
+            for (;;) {
+                const unsigned long long lo = s_before[wave][lane] * H;
+                const unsigned long long n = static_cast<unsigned long long>(stream_units(s_steps[wave][lane])) * H;
+                hit = __ballot(at >= lo && at - lo < n);
+                if (hit != 0) break;
+                base = uniform64(s_before[wave][63] + stream_units(s_steps[wave][63]));
+                b0 += 64;  // `at` is below the total: a later sequence holds it
+                chunk();
+            }
+            const uint32_t src = static_cast<uint32_t>(__builtin_ctzll(hit));
+            const uint32_t steps = __builtin_amdgcn_readfirstlane(s_steps[wave][src]);
+            const uint32_t units = stream_units(steps);
+            const unsigned long long off = at - uniform64(s_before[wave][src]) * H;  // below units * H
+            const uint32_t b = b0 + src;
+            const uint32_t h = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(off / units));
+            const uint32_t u0 = static_cast<uint32_t>(off - static_cast<unsigned long long>(h) * units);
+            const unsigned long long left = end - at;
+            const uint32_t u1 = left < units - u0 ? u0 + static_cast<uint32_t>(left) : units;
+            at += u1 - u0;
+            // units [u0, u1) of the pair: its steps follow the first kSegmentCost
+            if (u1 <= kSegmentCost) continue;
+            const uint32_t s0 = max(u0, kSegmentCost) - kSegmentCost;
+            const uint32_t n = u1 - kSegmentCost - s0;
+            const uint32_t per = (n + kWavesPerWg - 1) / kWavesPerWg;
+            const bool interleave = per == kInterleaveCpw;
+            const uint32_t skip = interleave ? wave : wave * per;
+            const uint32_t n_max = skip >= n ? 0u : interleave ? (n - skip + kWavesPerWg - 1) / kWavesPerWg : min(per, n - skip);
+            run_steps(b, h, 0u, s0 + skip, interleave ? kWavesPerWg : 1u, n_max,
+                      a.part + (static_cast<size_t>(blockIdx.x) + b * H + h) * rec);
+            __syncthreads();  // the next segment reuses the LDS
+        }
+    } else {
+        // One (sequence b, kv head h, split) of 4 waves x cpw steps per workgroup.
+        uint32_t split, h, b;
+        if (a.rowset_order) {
+            // Row sets of one sequence: items (kv head, split, row set), row sets fastest,
+            // each XCD (workgroup i runs on XCD i % 8) a contiguous range of them, so the
+            // workgroups an XCD runs together read the same keys (through its L2).  The
+            // grid is padded to a multiple of 8; items past a row set's splits exit.
+            const uint32_t total = a.max_splits * a.g.kv_heads * a.batch;
+            const uint32_t k = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+            if (k >= total) return;
+            b = k % a.batch;
+            split = (k / a.batch) % a.max_splits;
+            h = k / a.batch / a.max_splits;
+            if (a.count_ptr != nullptr && b >= *a.count_ptr) return;
+        } else {
+            const uint32_t bh = blockIdx.x / a.max_splits;
+            split = blockIdx.x % a.max_splits;
+            b = bh / geo.kv_heads;
+            h = bh % geo.kv_heads;
+        }
+        // Steps this wave may own, from the host bound alone: the first loads are issued
+        // before the context length arrives from memory.
+        const uint32_t cpw = a.cpw;
+        const uint32_t nsteps_max = (a.max_context + kChunk - 1) / kChunk;
+        const bool interleave = cpw == kInterleaveCpw;
+        const uint32_t stride = interleave ? kWavesPerWg : 1u;
+        const uint32_t first = interleave ? split * kWavesPerWg * cpw + wave : (split * kWavesPerWg + wave) * cpw;
+        const uint32_t last_excl = min(interleave ? (split + 1) * kWavesPerWg * cpw : first + cpw, nsteps_max);
+        const uint32_t n_max = first < last_excl ? (last_excl - first + stride - 1) / stride : 0;
+        run_steps(b, h, split, first, stride, n_max,
+                  a.part + ((static_cast<size_t>(b) * geo.kv_heads + h) * (a.max_splits + 1) + split) * rec);
+    }
 }
 
 
@@ -832,14 +860,15 @@ uint32_t resident_workgroups(uint32_t D, bool f32, uint32_t mode) {
 
 struct Plan {
     uint32_t cpw;
-    bool adaptive;  // steps per wave chosen on the device (launch_cpw)
     uint32_t splits;
     uint64_t counter_bytes;
     uint64_t part_bytes;
 };
 
 // rowsets: row sets of one sequence (a suffix run as decodes), all of about the same
-// length: the host plan is the launch's (no device-side choice), XCD-ordered.
+// length: XCD-ordered.  They all read the same keys: with long items the workgroups
+// running at once stream the same addresses together, so the steps per wave are capped
+// lower (exact suffix route at config 4: 1372 us at 64, 1000 at 32, 1055 at 16).
 Plan make_plan(const miikv_view* v, uint32_t q_heads, uint32_t batch, uint32_t max_context,
                uint32_t cpw_cap = 64, bool rowsets = false) {
     Plan p;
@@ -851,11 +880,9 @@ Plan make_plan(const miikv_view* v, uint32_t q_heads, uint32_t batch, uint32_t m
     // 23.0; 4k and 64k unchanged).  Batches keep the full target (config 3 is tuned so).
     const uint64_t target = (v->head_dim == 256 && batch == 1) ? kTargetWaves / 2 : kTargetWaves;
     uint64_t cpw = (waves + target - 1) / target;
-    // A batch: cpw is the floor of the device-side choice (launch_cpw), which
-    // can only raise it; the records and the grid are sized for the floor, a
-    // quarter of the all-sequences-full value.
+    // A batch: records for splits of a quarter of the all-sequences-full value, which the
+    // streamed plan (stream_workgroups) shares out.
     if (batch > 1 && !rowsets) cpw = (cpw + 3) / 4;
-    p.adaptive = batch > 1 && !rowsets;
     if (cpw < 1) cpw = 1;
     if (cpw > cpw_cap) cpw = cpw_cap;
     p.cpw = static_cast<uint32_t>(cpw);
@@ -867,6 +894,20 @@ Plan make_plan(const miikv_view* v, uint32_t q_heads, uint32_t batch, uint32_t m
     p.part_bytes = static_cast<uint64_t>(batch) * v->kv_heads * (p.splits + 1) * record_floats(G, v->head_dim) * 4;
     p.part_bytes = (p.part_bytes + 255) / 256 * 256;
     return p;
+}
+
+// Workgroups of the streamed plan (StreamTotal), 0 where it does not serve.  Its segments
+// are at most stream_wgs + batch * kv_heads - 1, and batch * kv_heads * splits record
+// slots hold them.  Launches whose splits all fit one resident round anyway are cut per
+// sequence (each wave then has the floor's one step in most cases; 4 sequences of up to
+// 1000 tokens, 32q/8kv/D128, 13.4 us either way), and so are sequences that are one split
+// each.  One round: with more workgroups than are resident the partial second round costs
+// more than it evens out (config 3, 512 resident: 448 / 512 / 640 / 1024 workgroups
+// 192 / 191 / 224 / 199 us).
+uint32_t stream_workgroups(const Plan& p, uint32_t batch, uint32_t kv_heads, uint32_t slots) {
+    const uint64_t bh = static_cast<uint64_t>(batch) * kv_heads;
+    if (batch == 1 || p.splits < 2 || bh * p.splits <= slots) return 0;
+    return static_cast<uint32_t>(std::min<uint64_t>(slots, bh * (p.splits - 1)));
 }
 
 }  // namespace
@@ -939,6 +980,15 @@ void launch_decode_t(dim3 grid, size_t lds, hipStream_t s, const SplitArgs& a) {
                                    dim3(64 * kWavesPerWg), lds, s, a);
             return;
         }
+    }
+    if (a.stream_wgs != 0) {
+        if (pair)
+            hipLaunchKernelGGL((decode_kernel<D, F32, APP, KF, VF, F32, false, true>), grid, dim3(64 * kWavesPerWg), lds,
+                               s, a);
+        else
+            hipLaunchKernelGGL((decode_kernel<D, F32, APP, KF, VF, false, false, true>), grid, dim3(64 * kWavesPerWg),
+                               lds, s, a);
+        return;
     }
     if (pair)
         hipLaunchKernelGGL((decode_kernel<D, F32, APP, KF, VF, F32>), grid, dim3(64 * kWavesPerWg), lds, s, a);
@@ -1041,12 +1091,6 @@ static miikv_status decode_impl(const miikv_view* view, const NewRows& rows,
     a.scale_log2 = scale * kLog2e;
     a.len_bstep = 0;
     a.count_ptr = nullptr;
-    // Row sets of one sequence all read the same keys: with long items the workgroups
-    // running at once stream the same addresses together, so the row-set route caps
-    // the steps per wave lower (host plan and device choice alike: the records are
-    // sized for the host's floor; exact suffix route at config 4: 1372 us at 64,
-    // 1000 at 32, 1055 at 16); decode batches of distinct sequences keep 64.
-    a.max_cpw = rs != nullptr ? kRowsetMaxCpw : 64u;
     a.rowset_order = rs != nullptr ? 1u : 0u;
     if (rs != nullptr) {  // row set b: len_add + b * pack (its last token's context)
         a.len_ptr = rs->len_ptr;
@@ -1088,12 +1132,15 @@ static miikv_status decode_impl(const miikv_view* view, const NewRows& rows,
     if (lds > 64 * 1024) return MIIKV_EUNSUPPORTED;
     // One workgroup per possible (sequence, kv head, split) work item, plus one per
     // (sequence, kv head) for the new token of the fused append.
-    uint64_t wgs = static_cast<uint64_t>(p.splits) * view->kv_heads * batch +
+    // (A streamed plan: its workgroups instead of the splits.)
+    const uint32_t slots = resident_workgroups(
+        view->head_dim, q_dtype == MIIKV_DTYPE_F32 && (view->head_dim == 128 || 2 * G > 16), view->quant_mode);
+    a.stream_wgs = rs != nullptr ? 0u : stream_workgroups(p, batch, view->kv_heads, slots);
+    uint64_t wgs = (a.stream_wgs != 0 ? a.stream_wgs : static_cast<uint64_t>(p.splits) * view->kv_heads * batch) +
                    (rows.any() ? static_cast<uint64_t>(view->kv_heads) * batch : 0);
     if (rs != nullptr) wgs = (wgs + 7) / 8 * 8;  // XCD-ordered items: a whole number of rounds over the XCDs
     if (wgs > 0x7fffffffu) return MIIKV_EINVAL;
     a.batch = batch;
-    a.slots = p.adaptive ? resident_workgroups(view->head_dim, q_dtype == MIIKV_DTYPE_F32 && (view->head_dim == 128 || 2 * G > 16), view->quant_mode) : 0u;
     const dim3 grid(static_cast<uint32_t>(wgs));
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool f32 = q_dtype == MIIKV_DTYPE_F32;

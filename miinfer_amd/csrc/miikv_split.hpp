@@ -33,12 +33,15 @@ struct SplitArgs {
     uint32_t cpw;         // chunks per wave
     uint32_t max_splits;  // splits per (sequence, kv head)
     uint32_t batch;       // sequences (row-sets)
-    uint32_t max_cpw;     // cap of the device-side steps per wave
-    // batch > 1: resident workgroups of the split kernel; the steps per wave are
-    // then chosen on the device from the lengths (at least cpw), 0: always cpw
-    uint32_t slots;
-    float* part;          // [batch][kv_heads][max_splits + 1][record]: the splits, then
-                          // with the fused append the new token's record at slot nsplit
+    // batch > 1, streamed plan: workgroups of the split kernel over which the batch's
+    // steps are cut evenly (stream_plan); 0: every (sequence, kv head) is cut by itself
+    // into splits of cpw steps per wave
+    uint32_t stream_wgs;
+    // [batch][kv_heads][max_splits + 1][record]: the splits, then with the fused append
+    // the new token's record at slot nsplit.  Streamed plan: segment records (StreamSeq)
+    // in the first batch * kv_heads * max_splits slots, then one slot per (sequence, kv
+    // head) for the new token.
+    float* part;
     float* out;
     const float* gate;
     float* gated_out;
@@ -69,32 +72,98 @@ __device__ __forceinline__ uint32_t split_length(const SplitArgs& a, uint32_t b)
     return L > a.max_context ? a.max_context : L;
 }
 
-// Steps per wave of a launch.  One sequence: the host's cpw.  A batch: the lengths
-// are only known on the device, so every workgroup of both kernels derives the
-// same value from them: the smallest cpw (>= the host's, which sized the records)
-// for which the work items, at most sum(L_b) * H / (4 waves * 32 * cpw) + count * H,
-// fit in one round of `slots` resident workgroups.  Called by every thread of the
-// workgroup (barriers inside); the first 256 threads do the sum.
-__device__ uint32_t launch_cpw(const SplitArgs& a) {
-    if (a.batch == 1 || a.slots == 0) return a.cpw;
-    __shared__ unsigned long long s_sum[256];
-    const uint32_t tid = threadIdx.x;
-    const uint32_t count = a.count_ptr ? min(a.batch, *a.count_ptr) : a.batch;
+// Streamed plan of a ragged batch.  The lengths are only known on the device, so every
+// wave derives the plan from them, by itself and without a barrier (a lane per sequence,
+// 64 sequences at a time).  In the order (sequence, kv head), every pair that holds keys
+// takes kSegmentCost units plus one per 32-key step on one axis, which is cut into
+// stream_wgs runs of `quota` units; workgroup w takes run w, which may cross from one pair
+// into the next: every workgroup of the one resident round has the same work whatever the
+// lengths are.  Each (workgroup, pair) with steps in common is a segment with a record of
+// its own, number w + pair: both only grow along the axis and no two segments share both,
+// so the numbers are distinct, and one pair's are consecutive.
+// Bound: the cache stream (HBM), then a segment's fixed latency (lengths, query, first
+// step, record), which kSegmentCost prices in steps.  Measured, fused append + attend, us,
+// against splits of one size per sequence that fit one round: 48 sequences of 64..4096
+// tokens, 32q/8kv/D128 (220 MB) 89.6 -> 48.3 (4.6 TB/s); 48 of 2080, 75.2 -> 47.3; 96 of
+// 500..1000, 24q/4kv/D256 66.0 -> 48.4; config 3 (1.18 GB) 192.0 -> 190.9.  kSegmentCost
+// 0 / 3 / 6 / 10 / 16 on the first: 58.9 / 50.8 / 48.3 / 49.1 / 49.7.
+#ifndef MIIKV_SEGMENT_COST
+#define MIIKV_SEGMENT_COST 6
+#endif
+constexpr uint32_t kSegmentCost = MIIKV_SEGMENT_COST;
+struct StreamTotal {
+    unsigned long long units;  // of one kv head, all sequences
+    unsigned long long quota;  // units per workgroup
+};
+
+// Keys of sequence b that the splits cover (the fused append's new token has a record of
+// its own), in 32-key steps.
+__device__ __forceinline__ uint32_t stream_steps(const SplitArgs& a, uint32_t b, uint32_t appended) {
+    const uint32_t L = split_length(a, b);
+    return (L - min(L, appended) + kChunk - 1) / kChunk;
+}
+__device__ __forceinline__ uint32_t stream_units(uint32_t steps) { return steps + (steps != 0 ? kSegmentCost : 0u); }
+
+__device__ __forceinline__ StreamTotal stream_total(const SplitArgs& a, uint32_t appended) {
+    const uint32_t lane = threadIdx.x & 63;
     unsigned long long sum = 0;
-    for (uint32_t bb = tid; bb < count && tid < 256; bb += 256) sum += split_length(a, bb);
-    if (tid < 256) s_sum[tid] = sum;
-    __syncthreads();
-    for (uint32_t off = 128; off > 0; off >>= 1) {
-        if (tid < off) s_sum[tid] += s_sum[tid + off];
-        __syncthreads();
+    for (uint32_t b = lane; b < a.batch; b += 64) sum += stream_units(stream_steps(a, b, appended));
+#pragma unroll
+    for (uint32_t off = 1; off < 64; off <<= 1) sum += __shfl_xor(sum, off, 64);
+    StreamTotal t;
+    t.units = sum;
+    // at least one step for each wave of a workgroup
+    const unsigned long long q = (sum * a.g.kv_heads + a.stream_wgs - 1) / a.stream_wgs;
+    t.quota = q < kWavesPerWg + kSegmentCost ? kWavesPerWg + kSegmentCost : q;
+    return t;
+}
+
+// This lane's sequence b0 + lane: its steps, and the units of one kv head before it given
+// those before b0.
+struct StreamSeq {
+    uint32_t steps;
+    unsigned long long before;
+};
+__device__ __forceinline__ StreamSeq stream_chunk(const SplitArgs& a, uint32_t b0, unsigned long long base,
+                                                  uint32_t appended) {
+    const uint32_t lane = threadIdx.x & 63;
+    StreamSeq s;
+    s.steps = b0 + lane < a.batch ? stream_steps(a, b0 + lane, appended) : 0u;
+    unsigned long long incl = stream_units(s.steps);
+#pragma unroll
+    for (uint32_t off = 1; off < 64; off <<= 1) {
+        const unsigned long long up = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += up;
     }
-    const unsigned long long total = s_sum[0] * a.g.kv_heads;
-    __syncthreads();  // s_sum is reused by the next call
-    const unsigned long long fixed_items = static_cast<unsigned long long>(count) * a.g.kv_heads;
-    const unsigned long long room = a.slots > fixed_items ? a.slots - fixed_items : a.slots;
-    const unsigned long long per = static_cast<unsigned long long>(kWavesPerWg) * kChunk * room;
-    const unsigned long long cpw = (total + per - 1) / per;
-    return static_cast<uint32_t>(cpw < a.cpw ? a.cpw : (cpw > a.max_cpw ? a.max_cpw : cpw));
+    s.before = base + incl - stream_units(s.steps);
+    return s;
+}
+
+// Records of (sequence b, kv head h): `first` and `count` (the new token's record not
+// counted).  b and h may differ between the lanes of a wave; every lane takes part.
+__device__ __forceinline__ void stream_records(const SplitArgs& a, uint32_t b, uint32_t h, uint32_t appended,
+                                               uint32_t& first, uint32_t& count) {
+    const StreamTotal t = stream_total(a, appended);
+    unsigned long long base = 0, before = 0;
+    uint32_t steps = 0;
+    for (uint32_t b0 = 0; b0 < a.batch; b0 += 64) {
+        const StreamSeq s = stream_chunk(a, b0, base, appended);
+        const unsigned long long bf = __shfl(s.before, b & 63, 64);
+        const uint32_t st = __shfl(s.steps, b & 63, 64);
+        if (b - b0 < 64) {
+            before = bf;
+            steps = st;
+        }
+        base = __shfl(s.before, 63, 64) + stream_units(__shfl(s.steps, 63, 64));
+    }
+    first = count = 0;
+    if (steps == 0) return;
+    // the pair's steps follow its kSegmentCost units
+    const unsigned long long start = before * a.g.kv_heads + static_cast<unsigned long long>(h) * stream_units(steps) + kSegmentCost;
+    const uint32_t w0 = static_cast<uint32_t>(start / t.quota);
+    const uint32_t w1 = static_cast<uint32_t>((start + steps - 1) / t.quota);
+    first = w0 + b * a.g.kv_heads + h;
+    count = w1 - w0 + 1;
 }
 
 // Split count of sequence b at `cpw` steps per wave (0 when L == 0).
@@ -129,6 +198,40 @@ __device__ __forceinline__ void merge_state(float& m, float& l, float4& acc, flo
     acc.y = acc.y * f1 + a2.y * f2;
     acc.z = acc.z * f1 + a2.z * f2;
     acc.w = acc.w * f1 + a2.w * f2;
+}
+
+// Record slots of one (sequence b, kv head h): `first` on, and how many may be read before
+// the count is known.  Streamed plan: the segments' records, then the new token's.
+struct CombineRecords {
+    size_t first;
+    size_t appended;   // streamed plan: slot of the new token's record
+    uint32_t nseg;     // streamed plan: segments (the other plan: all slots)
+    uint32_t slots;
+    __device__ __forceinline__ const float* at(const SplitArgs& a, uint32_t j, uint32_t rec) const {
+        return a.part + (j < nseg ? first + j : appended) * rec;
+    }
+};
+__device__ __forceinline__ CombineRecords combine_records(const SplitArgs& a, uint32_t b, uint32_t h, uint32_t bh,
+                                                          bool append) {
+    CombineRecords r;
+    if (a.stream_wgs == 0) {
+        r.nseg = r.slots = a.max_splits + 1;
+        r.first = static_cast<size_t>(bh) * r.slots;
+        r.appended = r.first;
+        return r;
+    }
+    uint32_t first;
+    stream_records(a, b, h, append ? 1u : 0u, first, r.nseg);
+    r.first = first;
+    r.appended = static_cast<size_t>(a.batch) * a.g.kv_heads * a.max_splits + bh;
+    r.slots = r.nseg + (append && split_length(a, b) > 0 ? 1u : 0u);
+    return r;
+}
+// Records of sequence b (the plan of fixed splits waits for its length here).
+__device__ __forceinline__ uint32_t combine_count(const SplitArgs& a, uint32_t b, const CombineRecords& r, bool append) {
+    if (a.stream_wgs != 0) return r.slots;
+    const uint32_t L = split_length(a, b);
+    return split_count(L, a.cpw) + (append && L > 0 ? 1u : 0u);
 }
 
 // Gate values of elements i..i+3.  Called after the record loads are issued: a load
@@ -205,8 +308,8 @@ __global__ void __launch_bounds__(256) combine_kernel(SplitArgs a) {
     const size_t out_row0 = ((static_cast<size_t>(b) * a.pack + tp) * a.q_heads + static_cast<size_t>(h) * Gt +
                              (hn - tp * Gt)) * D - static_cast<size_t>(hn) * D;
     const uint32_t rec = record_floats(G, D);
-    const uint32_t slots = a.max_splits + 1;
-    const float* part = a.part + (static_cast<size_t>(bh) * slots) * rec;
+    const CombineRecords R = combine_records(a, b, h, bh, APPEND);
+    const uint32_t slots = R.slots;
 
     constexpr uint32_t kSpec = 3;
     float ms[kSpec], ls[kSpec];
@@ -218,7 +321,7 @@ __global__ void __launch_bounds__(256) combine_kernel(SplitArgs a) {
         ls[j] = 0.0f;
         vv[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if (sp < slots) {
-            const float* r = part + static_cast<size_t>(sp) * rec;
+            const float* r = R.at(a, sp, rec);
             ms[j] = r[GD + hn];
             ls[j] = r[GD + G + hn];
             vv[j] = *reinterpret_cast<const float4*>(r + e);
@@ -226,10 +329,8 @@ __global__ void __launch_bounds__(256) combine_kernel(SplitArgs a) {
     }
     float gv[4];
     combine_gate(a, out_row0 + e, gv);
-    const uint32_t cpw = launch_cpw(a);
     if (a.count_ptr != nullptr && b >= *a.count_ptr) return;
-    const uint32_t L = split_length(a, b);
-    const uint32_t nrec = split_count(L, cpw) + (APPEND && L > 0 ? 1u : 0u);
+    const uint32_t nrec = combine_count(a, b, R, APPEND);
 
     float m = -INFINITY, l = 0.0f;
     float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -237,7 +338,7 @@ __global__ void __launch_bounds__(256) combine_kernel(SplitArgs a) {
     for (uint32_t j = 0; j < kSpec; ++j)
         if (rg + 32 * j < nrec) merge_state(m, l, acc, ms[j], ls[j], vv[j]);
     for (uint32_t sp = rg + 32 * kSpec; sp < nrec; sp += 32) {
-        const float* r = part + static_cast<size_t>(sp) * rec;
+        const float* r = R.at(a, sp, rec);
         merge_state(m, l, acc, r[GD + hn], r[GD + G + hn], *reinterpret_cast<const float4*>(r + e));
     }
     // Butterfly over the 8 record groups of this wave (lanes 8, 16, 32 apart).
@@ -291,16 +392,17 @@ __global__ void __launch_bounds__(256) combine_narrow_kernel(SplitArgs a) {
     const size_t out_row0 = ((static_cast<size_t>(b) * a.pack + tp) * a.q_heads + static_cast<size_t>(h) * Gt +
                              (hn - tp * Gt)) * D - static_cast<size_t>(hn) * D;
     const uint32_t rec = record_floats(G, D);
-    const float* part = a.part + (static_cast<size_t>(bhc) * (a.max_splits + 1)) * rec;
+    const CombineRecords R = combine_records(a, b, h, bhc, APPEND);
     // The first batch of record slots is read before the context length arrives (slots
-    // past the row set's count hold stale bytes and are dropped below), then the gate.
-    const uint32_t slots = a.max_splits + 1;
+    // past the row set's count hold stale bytes and are dropped below; a streamed plan
+    // has its count already), then the gate.
+    const uint32_t slots = R.slots;
     float ms[kNarrowRecords], ls[kNarrowRecords];
     float4 vv[kNarrowRecords];
 #pragma unroll
     for (uint32_t j = 0; j < kNarrowRecords; ++j) {
         if (j < slots) {
-            const float* r = part + static_cast<size_t>(j) * rec;
+            const float* r = R.at(a, j, rec);
             ms[j] = r[GD + hn];
             ls[j] = r[GD + G + hn];
             vv[j] = *reinterpret_cast<const float4*>(r + e);
@@ -308,13 +410,10 @@ __global__ void __launch_bounds__(256) combine_narrow_kernel(SplitArgs a) {
     }
     float gv[4];
     combine_gate(a, out_row0 + e, gv);
-    // steps per wave (every thread of the workgroup takes part) with the loads in flight
-    const uint32_t cpw = launch_cpw(a);
     // a whole 32-value block shares b (GD is a multiple of 32), so the 8 threads of a
     // block take the same exit
     if (a.count_ptr != nullptr && b >= *a.count_ptr) return;
-    const uint32_t L = split_length(a, b);
-    const uint32_t nrec = split_count(L, cpw) + (APPEND && L > 0 ? 1u : 0u);
+    const uint32_t nrec = combine_count(a, b, R, APPEND);
     float m = -INFINITY, l = 0.0f;
     float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
@@ -325,7 +424,7 @@ __global__ void __launch_bounds__(256) combine_narrow_kernel(SplitArgs a) {
         for (uint32_t j = 0; j < kNarrowRecords; ++j) {
             ms[j] = -INFINITY;
             if (sp0 + j < nrec) {
-                const float* r = part + static_cast<size_t>(sp0 + j) * rec;
+                const float* r = R.at(a, sp0 + j, rec);
                 ms[j] = r[GD + hn];
                 ls[j] = r[GD + G + hn];
                 vv[j] = *reinterpret_cast<const float4*>(r + e);

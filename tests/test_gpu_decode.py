@@ -450,3 +450,41 @@ def test_decode_random_batches(gpu, seed):
         assert_attention_close(out[s], expect, f"{what} seq {s} L={n}")
         if gate is not None:
             assert_attention_close(gated[s].cpu().numpy(), expect / (1 + np.exp(-gate[s])), f"{what} gated seq {s}")
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("hq,hk,d,f32", [(16, 4, 128, False), (24, 4, 256, True)])
+def test_decode_streamed_batch_edges(gpu, hq, hk, d, f32, fused):
+    """More sequences than a wave has lanes (the streamed plan takes 64 at a time), empty
+    ones, single keys, step and page edges: the runs cross sequences and kv heads at every
+    offset.  Every row against the oracle (fused: the new token's row among the keys)."""
+    import miinfer_amd as m
+    rng = np.random.default_rng(5)
+    edges = [0, 1, 2, 31, 32, 33, 64, 65, 127, 128, 129, 255, 256, 257, 511, 513, 700, 768]
+    lens = np.array((edges * 4 + [768, 1])[:70], np.int32)
+    pt, stride = 256, 3
+    table = rng.permutation(lens.size * stride).astype(np.int32).reshape(lens.size, stride)
+    cache = m.KvCache.paged_cache(hk, d, table.size, _dev(table, gpu), page_tokens=pt)
+    refs = []
+    k_new = np.zeros((lens.size, hk, d), np.float16)
+    v_new = np.zeros((lens.size, hk, d), np.float16)
+    for s, n in enumerate(lens.tolist()):
+        k = randn_f16(rng, (n, hk, d))
+        v = randn_f16(rng, (n, hk, d))
+        stored = max(n - 1, 0) if fused else n
+        if stored:
+            cache.append(_dev(k[:stored], gpu), _dev(v[:stored], gpu), base_position=0, seq=s)
+        if n:
+            k_new[s], v_new[s] = k[-1], v[-1]
+        refs.append(oracle.quantize_rows(k.transpose(1, 0, 2)) + oracle.quantize_rows(v.transpose(1, 0, 2)))
+    q = rng.standard_normal((lens.size, hq, d)).astype(np.float32) if f32 else randn_f16(rng, (lens.size, hq, d))
+    new = {"k_new": _dev(k_new, gpu), "v_new": _dev(v_new, gpu)} if fused else {}
+    out, _ = m.decode_attention(cache, _dev(q, gpu), lengths=_dev(lens, gpu), max_context=stride * pt, **new)
+    torch.cuda.synchronize()
+    out = out.cpu().numpy()
+    for s, n in enumerate(lens.tolist()):
+        if n == 0:
+            assert not out[s].any()
+            continue
+        expect = oracle.attention_q8(q[s].astype(np.float32), *refs[s], n, hq, 1 / math.sqrt(d))
+        assert_attention_close(out[s], expect, f"seq {s} L={n}")
