@@ -27,7 +27,9 @@ SOURCES = [
 # Per-source code-generation options.  The suffix kernel keeps its MFMA
 # accumulators in architectural VGPRs (see the note in miikv_suffix.hip).
 SOURCE_FLAGS = {
-    "miikv_suffix.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    # Its step loops start on 64-byte boundaries: where they fall by chance moved config 4
+    # by 1% (135.4 / 137.0 us).
+    "miikv_suffix.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-falign-loops=64"],
     # The split-K decode kernels are scheduled for instruction-level parallelism
     # (config 2 at 32k: 20.2 -> 19.8 us per layer-token; config 3 unchanged; the
     # suffix kernel measured no better with it, so it keeps the default).

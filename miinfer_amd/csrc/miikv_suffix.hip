@@ -238,18 +238,22 @@ __global__ void __launch_bounds__(256) expand_kernel(ExpandArgs a) {
 // (-amdgpu-mfma-vgpr-form): at D = 256 a wave holds O^T (128 registers), the
 // query fragments (64), S^T (16) and the softmax working set, and within the 256
 // registers of two waves per SIMD the lazy rescale multiplies O^T in place.
-#ifndef MIIKV_SUFFIX_STAGGER
-#define MIIKV_SUFFIX_STAGGER 1
-#endif
-constexpr bool kSufStagger = MIIKV_SUFFIX_STAGGER != 0;
-// Prefetch distance in steps (config 4, same box: 1 and 3 both ~1-2 us slower
-// than 2; 3 takes all 160 KB of LDS).
-#ifndef MIIKV_SUFFIX_DIST
-#define MIIKV_SUFFIX_DIST 2
-#endif
-constexpr uint32_t kDist = MIIKV_SUFFIX_DIST;
-constexpr uint32_t kSufBufs = kSufStagger ? kDist + 2 : kDist + 1;  // LDS tile buffers
-
+//
+// The 8-wave form (kSufWaves) runs the two waves of a SIMD half a step apart and fetches
+// two steps ahead (config 4, same box: 1 and 3 steps both ~1-2 us slower than 2; 3 takes
+// all 160 KB of LDS).  The 4-wave form (kSufWavesSmall) has two buffers, so two workgroups
+// share a CU (or one runs alone in a small launch), each fetching one step ahead with
+// copies that the barrier does not drain and reading its LDS fragments one pair of MFMAs
+// ahead.  Its waves are less often held by a workgroup's slowest: a step with one
+// workgroup per CU takes ~1.2 us at D = 256 against ~1.8 in the 8-wave form.  (The same
+// two changes in the 8-wave form: config 4 level, D = 128 5-10% slower.)
+template <uint32_t NW>
+struct SuffixForm {
+    static constexpr bool stagger = NW == kSufWaves;
+    static constexpr bool ahead = NW == kSufWavesSmall;  // counted copies, fragments read ahead
+    static constexpr uint32_t dist = NW == kSufWaves ? 2 : 1;             // prefetch distance in steps
+    static constexpr uint32_t bufs = stagger ? dist + 2 : dist + 1;       // LDS tile buffers
+};
 
 // The softmax keeps its VALU count low (v_max3 row max, v_dot2 row sum): VALU work
 // of the two waves of a SIMD hides only partly under their MFMAs.
@@ -260,13 +264,41 @@ __device__ __forceinline__ float max3_raw(float x, float y, float z) {
     return r;
 }
 
-template <uint32_t D>
-__global__ void __launch_bounds__(64 * kSufWaves) suffix_kernel(SuffixArgs a) {
+// `use`(c, fragment c) for c < N, fragment c at `t` + 512 * c in LDS (this lane's 8 halves).
+// AHEAD: the next pair of fragments is on its way while a pair's MFMAs run.
+template <uint32_t N, bool AHEAD, typename F>
+__device__ __forceinline__ void mfma_pairs(const _Float16* t, F use) {
+    if constexpr (!AHEAD) {
+#pragma unroll
+        for (uint32_t c = 0; c < N; ++c) use(c, *reinterpret_cast<const half8*>(t + 512 * c));
+    } else {
+        half8 f[2][2];
+        f[0][0] = *reinterpret_cast<const half8*>(t);
+        f[0][1] = *reinterpret_cast<const half8*>(t + 512);
+#pragma unroll
+        for (uint32_t c = 0; c < N; c += 2) {
+            const uint32_t k = (c / 2) & 1;
+            if (c + 2 < N) {
+                f[k ^ 1][0] = *reinterpret_cast<const half8*>(t + 512 * (c + 2));
+                f[k ^ 1][1] = *reinterpret_cast<const half8*>(t + 512 * (c + 3));
+            }
+            __builtin_amdgcn_sched_barrier(0);  // the scheduler would sink the reads to their use
+            use(c, f[k][0]);
+            use(c + 1, f[k][1]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+}
+
+template <uint32_t D, uint32_t NW>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) suffix_kernel(SuffixArgs a) {
+    using Form = SuffixForm<NW>;
+    constexpr uint32_t kDist = Form::dist, kSufBufs = Form::bufs, kRows = 32 * NW;
     constexpr uint32_t NB = D / 32;         // PV M-tiles
     constexpr uint32_t NC = D / 16;         // QK k-chunks (K fragments)
     constexpr uint32_t TILE = tile_halves(D);
     constexpr uint32_t CHUNKS = TILE * 2 / 1024;  // 1 KiB copy chunks per step
-    static_assert(CHUNKS % kSufWaves == 0, "copy chunks must split evenly over waves");
+    static_assert(CHUNKS % NW == 0, "copy chunks must split evenly over waves");
     __shared__ __align__(16) _Float16 s_t[kSufBufs][TILE];
     // The tile buffers are the kernel's whole LDS.  Measured at D = 256: 8 bytes of
     // LDS beyond 128 KiB (two flags) slowed the step loop by ~12%, so any other LDS
@@ -281,17 +313,14 @@ __global__ void __launch_bounds__(64 * kSufWaves) suffix_kernel(SuffixArgs a) {
     }
     const uint32_t G = a.group;
     // XCD-aware order: workgroup L runs on XCD L % 8.  Each XCD gets an equal,
-    // contiguous range of the (group, row block) sequence, group-major, so the
-    // row blocks of one (kv head, split) group, which read the same tiles, share
-    // an L2; with rows_together the sequence is (kv head, row block, split).  The
-    // grid is padded to a multiple of 8 workgroups.
+    // contiguous range of the items in a.order's sequence: what its workgroups share (the
+    // tiles of a (kv head, split), the query rows of a row block) they read through one
+    // L2.  The grid is padded to a multiple of 8 workgroups.
     const uint32_t L = blockIdx.x;
     const uint32_t per_xcd = gridDim.x / 8;
     const uint32_t idx = (L % 8) * per_xcd + L / 8;
     uint32_t h, split, rb;
-    if (a.rows_together) {
-        // the splits of one row block next to each other: an XCD's workgroups share
-        // their query rows through its L2 (and each tile range among fewer of them)
+    if (a.order == kSufRowsTogether) {
         const uint32_t gi = idx / a.splits;
         split = idx % a.splits;
         h = gi / a.row_blocks;
@@ -303,6 +332,8 @@ __global__ void __launch_bounds__(64 * kSufWaves) suffix_kernel(SuffixArgs a) {
         h = grp % a.g.kv_heads;
         split = grp / a.g.kv_heads;
         rb = idx % a.row_blocks;
+        if (a.order == kSufLongFirst || (a.order == kSufPaired && rb < a.row_blocks / 2)) rb = a.row_blocks - 1 - rb;
+        else if (a.order == kSufPaired) rb -= a.row_blocks / 2;
     }
     const uint32_t tid = threadIdx.x;
     const uint32_t wave = tid >> 6;
@@ -310,7 +341,7 @@ __global__ void __launch_bounds__(64 * kSufWaves) suffix_kernel(SuffixArgs a) {
     const uint32_t n = lane & 31;
     const uint32_t hh = lane >> 5;
     const uint32_t rows = T * G;
-    const uint32_t r0 = rb * kSufRows;
+    const uint32_t r0 = rb * kRows;
     if (r0 >= rows) return;
 
     const uint32_t row = r0 + wave * 32 + n;
@@ -321,7 +352,7 @@ __global__ void __launch_bounds__(64 * kSufWaves) suffix_kernel(SuffixArgs a) {
     // Smallest limit among this wave's rows: steps wholly at or below it need no mask.
     const uint32_t wave_lim = P + min(r0 + wave * 32, rows - 1) / G;
 
-    const uint32_t last_row = min(r0 + kSufRows, rows) - 1;
+    const uint32_t last_row = min(r0 + kRows, rows) - 1;
     const uint32_t nkeys = P + last_row / G + 1;
     const uint32_t key_lo = split * a.split_keys;
     if (key_lo >= nkeys) return;  // no row of this workgroup has keys in this split
@@ -367,15 +398,17 @@ __global__ void __launch_bounds__(64 * kSufWaves) suffix_kernel(SuffixArgs a) {
     }
 
     // Step s's tile into LDS buffer b: CHUNKS KiB, each wave copying every
-    // kSufWaves-th KiB with one 16-byte direct-to-LDS load per lane.
+    // NW-th KiB with one 16-byte direct-to-LDS load per lane.
     const char* tiles_h = reinterpret_cast<const char*>(a.tiles + static_cast<size_t>(h) * a.steps * TILE);
     auto fetch = [&](uint32_t s, uint32_t b) {
         const char* src = tiles_h + static_cast<size_t>(s) * TILE * 2 + lane * 16;
         char* dst = reinterpret_cast<char*>(s_t[b]);
+        const uint32_t dst_off = lds_offset(s_t) + b * (TILE * 2);
 #pragma unroll
-        for (uint32_t u = 0; u < CHUNKS / kSufWaves; ++u) {
-            const uint32_t chunk = wave + kSufWaves * u;
-            __builtin_amdgcn_global_load_lds(src + chunk * 1024, dst + chunk * 1024, 16, 0, 0);
+        for (uint32_t u = 0; u < CHUNKS / NW; ++u) {
+            const uint32_t chunk = wave + NW * u;
+            if constexpr (Form::ahead) copy_to_lds(src + chunk * 1024, dst_off + chunk * 1024);
+            else __builtin_amdgcn_global_load_lds(src + chunk * 1024, dst + chunk * 1024, 16, 0, 0);
         }
     };
 
@@ -388,20 +421,25 @@ __global__ void __launch_bounds__(64 * kSufWaves) suffix_kernel(SuffixArgs a) {
     // Step s lives in buffer s % kSufBufs; the fetch of step s + kDist is issued at
     // the top of step s into a buffer that no wave reads any more (the barrier that
     // ends each step orders it after those reads).
-    constexpr uint32_t kPer = CHUNKS / kSufWaves;  // loads per wave per fetch
+    constexpr uint32_t kPer = CHUNKS / NW;  // loads per wave per fetch
     for (uint32_t k = 0; k < kDist; ++k)
         if (s_begin + k < s_end) fetch(s_begin + k, (s_begin + k) % kSufBufs);
     // the query and the first step's tile; the later prefetches may stay in flight
     if (kDist > 1 && s_begin + 1 < s_end) wait_vmem_le<(kDist - 1) * kPer>();
     else wait_vmem();
-    __syncthreads();
+    auto barrier = [&]() __attribute__((always_inline)) {
+        if constexpr (Form::ahead) lds_barrier();
+        else __syncthreads();
+    };
+    barrier();
 
     // ---- S^T = K^ Q^T of step s
     auto scores = [&](uint32_t s) __attribute__((always_inline)) {
         const _Float16* tk = s_t[s % kSufBufs] + lane * 8;
         float16v acc = {};
-#pragma unroll
-        for (uint32_t c = 0; c < NC; ++c) acc = mfma_32x32x16(*reinterpret_cast<const half8*>(tk + 512 * c), qf[c], acc);
+        mfma_pairs<NC, Form::ahead>(tk, [&](uint32_t c, half8 f) __attribute__((always_inline)) {
+            acc = mfma_32x32x16(f, qf[c], acc);
+        });
         return acc;
     };
     // ---- online softmax over this lane's 16 keys of row n; P^T fragments out
@@ -451,11 +489,9 @@ __global__ void __launch_bounds__(64 * kSufWaves) suffix_kernel(SuffixArgs a) {
     // ---- O^T += V^T P^T of step s
     auto values = [&](uint32_t s, const half8 (&pb)[2]) __attribute__((always_inline)) {
         const _Float16* tv = s_t[s % kSufBufs] + 64 * 8 * NC + lane * 8;
-#pragma unroll
-        for (uint32_t mt = 0; mt < NB; ++mt)
-#pragma unroll
-            for (uint32_t kc = 0; kc < 2; ++kc)
-                O[mt] = mfma_32x32x16(*reinterpret_cast<const half8*>(tv + 512 * (2 * mt + kc)), pb[kc], O[mt]);
+        mfma_pairs<2 * NB, Form::ahead>(tv, [&](uint32_t f, half8 v) __attribute__((always_inline)) {
+            O[f / 2] = mfma_32x32x16(v, pb[f % 2], O[f / 2]);
+        });
     };
     // Top of step s: the fetch of step s + kDist.  End of step s: step s+1's tile
     // must have landed (this step's own fetch may stay in flight), then the barrier.
@@ -465,17 +501,17 @@ __global__ void __launch_bounds__(64 * kSufWaves) suffix_kernel(SuffixArgs a) {
     auto step_end = [&](uint32_t s) __attribute__((always_inline)) {
         if (s + kDist < s_end) wait_vmem_le<(kDist > 1 ? kPer : 0)>();
         else wait_vmem();
-        __syncthreads();
+        barrier();
     };
 
-    // With kSufStagger the two waves of each SIMD (waves w and w + kSufWaves/2)
+    // With Form::stagger the two waves of each SIMD (waves w and w + NW/2)
     // run half a step apart: the leading half orders a step as scores, softmax,
     // values; the lagging half adds step s-1's values before step s's scores, so
     // one wave's softmax can overlap the other's MFMAs (C4: ~2% faster).
     // Every wave still passes one barrier per step; the lagging half's values of
     // step s-1 read a buffer that is refilled only at the top of step s+1
     // (kSufBufs >= kDist + 2).
-    const bool lag = kSufStagger && wave >= kSufWaves / 2;
+    const bool lag = Form::stagger && wave >= NW / 2;
     if (!lag) {
         for (uint32_t s = s_begin; s < s_end; ++s) {
             step_begin(s);
@@ -1038,11 +1074,13 @@ struct SuffixPlan {
 // 256 keys per split).  Monotone in key_bound, so a plan made with the cache
 // capacity covers any smaller context.
 // exact: the plan of suffix_exact_kernel (its tiles and its rows per workgroup).
+// waves: the form of suffix_kernel (or suffix_exact_kernel's).
 SuffixPlan make_suffix_plan(const miikv_view* v, uint32_t q_heads, uint32_t tokens, uint64_t key_bound,
-                            bool allow_split, uint64_t stride_bound = 0, bool exact = false) {
+                            bool allow_split, uint64_t stride_bound = 0, bool exact = false,
+                            uint32_t waves = kSufWaves) {
     SuffixPlan p{1, 0, 0, 0, 0};
     const uint32_t G = q_heads / v->kv_heads;
-    const uint32_t rows_per_wg = exact ? kExRows : kSufRows;
+    const uint32_t rows_per_wg = exact ? kExRows : 32 * waves;
     // the tile area holds stride_bound keys per kv head (the capacity for incremental
     // tiles, whose layout must not move between calls), the splits cover key_bound
     p.steps = static_cast<uint32_t>((std::max(key_bound, stride_bound) + kSufStep - 1) / kSufStep);
@@ -1054,9 +1092,11 @@ SuffixPlan make_suffix_plan(const miikv_view* v, uint32_t q_heads, uint32_t toke
     const uint64_t wgs = (static_cast<uint64_t>(tokens) * G + rows_per_wg - 1) / rows_per_wg * v->kv_heads;
     // Splits: as many as keep every workgroup resident in one round (the
     // per-workgroup cost does not shrink with more concurrent workgroups, so a
-    // second partial round costs a full one), at least 256 keys each.
-    const uint64_t by_keys = std::min<uint64_t>((key_bound + 255) / 256, kSufMaxSplits);
-    uint64_t want = std::max<uint64_t>(1, kSufSlots / wgs);
+    // second partial round costs a full one), at least kSufMinKeys keys each; the 4-wave
+    // form is split to one workgroup per CU (suffix_form).
+    const uint64_t min_keys = waves == kSufWaves ? kSufMinKeys : kSufMinKeysSmall;
+    const uint64_t by_keys = std::min<uint64_t>((key_bound + min_keys - 1) / min_keys, kSufMaxSplits);
+    uint64_t want = std::max<uint64_t>(1, kSufResidentWaves / kSufWaves / wgs);
     want = std::max<uint64_t>(1, std::min<uint64_t>({want, by_keys, kSufMaxSplits}));
     if (want <= 1) return p;
     const uint64_t unit = kSufStep;
@@ -1069,6 +1109,29 @@ SuffixPlan make_suffix_plan(const miikv_view* v, uint32_t q_heads, uint32_t toke
     // Records sized for `want` (>= splits): a plan for a shorter context never needs more.
     p.part_bytes = want * v->kv_heads * tokens * G * (exact ? 4 * v->head_dim + 8 : part_row_bytes(v->head_dim));
     return p;
+}
+
+// Waves per workgroup of suffix_kernel for a suffix of `tokens` tokens at position `base`
+// (UINT32_MAX: on the device) with keys below key_bound.
+// The 4-wave form runs a step in about 2/3 of the 8-wave form's time where it has a CU to
+// itself, for half the rows: it pays in launches that leave CUs idle otherwise.  Two of its
+// workgroups on a CU are 4-7% behind one 8-wave workgroup, so it serves no larger launch,
+// but for one: an unsplit launch whose causal rows make the workgroups unequal (the first
+// rows see `base` keys, the last base + tokens) pairs long with short ones on each CU.
+// Measured, us, 8 waves -> 4: 24q/4kv/D256, 77 tokens over 3001 49.4 -> 39.2; 128 over 0 /
+// 1000 / 4000 32.3 -> 25.3 / 44.6 -> 35.5 / 53.6 -> 53.8; 512 over 0 48.3 -> 39.6, over 8192
+// 136.5 -> 142.5; 2048 over 0 (unsplit) 122.2 -> 111.4; 32q/8kv/D128, 128 over 1000 30.3 ->
+// 26.3, 2048 over 0 72.2 -> 62.7, 2000 over 1000 107.9 -> 98.2.
+uint32_t suffix_form(const miikv_view* v, uint32_t q_heads, uint32_t tokens, uint64_t key_bound, uint32_t base) {
+    const uint64_t cus = kSufResidentWaves / kSufWaves;
+    const uint64_t rows = static_cast<uint64_t>(tokens) * (q_heads / v->kv_heads);
+    const uint64_t rows_small = 32 * kSufWavesSmall;
+    const uint64_t wgs = (rows + rows_small - 1) / rows_small * v->kv_heads;
+    const SuffixPlan big = make_suffix_plan(v, q_heads, tokens, key_bound, true);
+    if (big.splits == 1 && wgs > cus)
+        return wgs <= 2 * cus && base <= tokens ? kSufWavesSmall : kSufWaves;
+    const SuffixPlan small = make_suffix_plan(v, q_heads, tokens, key_bound, big.splits > 1, 0, false, kSufWavesSmall);
+    return wgs * small.splits <= cus && 2ull * small.split_keys <= 3ull * big.split_keys ? kSufWavesSmall : kSufWaves;
 }
 
 }  // namespace
@@ -1088,7 +1151,8 @@ extern "C" uint64_t miikv_suffix_workspace_bytes(const miikv_view* view, uint32_
         suffix_runs_as_decode(view, q_heads, token_count, true))
         dec = suffix_by_decode_bytes(view, q_heads, token_count, static_cast<uint32_t>(std::min<uint64_t>(cap, 0xffffffffu)));
     const SuffixPlan p = make_suffix_plan(view, q_heads, token_count, cap, true);
-    return p.tile_bytes + std::max(dec, p.part_bytes);
+    const SuffixPlan small = make_suffix_plan(view, q_heads, token_count, cap, true, 0, false, kSufWavesSmall);
+    return p.tile_bytes + std::max({dec, p.part_bytes, small.part_bytes});
 }
 
 // Exact route: the tiles (kept for MIIKV_SUFFIX_TILES_CURRENT, whose decode-route
@@ -1159,8 +1223,7 @@ static miikv_status suffix_impl(const miikv_view* view, const uint16_t* k_new, c
     const uint64_t cap = view_seq_capacity(view);
     if (prefill_state == nullptr && static_cast<uint64_t>(base_position) + token_count > cap) return MIIKV_EINVAL;
     const uint64_t rows = static_cast<uint64_t>(token_count) * G;
-    const uint64_t blocks = (rows + kSufRows - 1) / kSufRows;
-    if (blocks > 0x7fffffffu || static_cast<uint64_t>(token_count) * view->kv_heads > 0x7fffffffu)
+    if ((rows + 31) / 32 > 0x7fffffffu || static_cast<uint64_t>(token_count) * view->kv_heads > 0x7fffffffu)
         return MIIKV_EINVAL;
     // The key bound: the known context (host base position) or the capacity (device
     // state).  A workspace of miikv_suffix_workspace_bytes() bytes always suffices;
@@ -1286,11 +1349,18 @@ static miikv_status suffix_impl(const miikv_view* view, const uint16_t* k_new, c
                                 bound32, out, gate, gated_out, static_cast<uint8_t*>(workspace) + dec_off,
                                 workspace_bytes - dec_off, stream);
     }
-    SuffixPlan plan = make_suffix_plan(view, q_heads, token_count, bound, true, stride_bound);
+    const SuffixPlan big = make_suffix_plan(view, q_heads, token_count, bound, true, stride_bound);
+    uint32_t waves = suffix_form(view, q_heads, token_count, bound, prefill_state ? UINT32_MAX : base_position);
+    // (a launch that the 8-wave form does not split is not split: split records are fp16)
+    SuffixPlan plan = waves == kSufWaves ? big
+                                         : make_suffix_plan(view, q_heads, token_count, bound, big.splits > 1,
+                                                            stride_bound, false, waves);
     if (workspace_bytes < plan.total()) {
-        plan = tile_plan;
+        waves = kSufWaves;
+        plan = workspace_bytes < big.total() ? tile_plan : big;
         if (workspace_bytes < plan.total()) return MIIKV_EWORKSPACE;
     }
+    const uint64_t blocks = (rows + 32 * waves - 1) / (32 * waves);
     if (plan.steps > 65535u * 64u) return MIIKV_EINVAL;
 
     expand(plan, k_new != nullptr);
@@ -1318,13 +1388,20 @@ static miikv_status suffix_impl(const miikv_view* view, const uint16_t* k_new, c
     // split: 135.0 -> 131.7 us; the ladder at P = 4096 3.5% faster); long ones keep
     // the (kv head, split)-major order, whose tiles more row blocks share (P = 65536:
     // 0.3% slower the other way, P = 32768 level).
-    a.rows_together = plan.splits > 1 && plan.split_keys <= 128 * kSufStep ? 1u : 0u;
+    if (plan.splits > 1) a.order = plan.split_keys <= 128 * kSufStep ? kSufRowsTogether : kSufTilesTogether;
+    else a.order = waves == kSufWavesSmall && static_cast<uint64_t>(view->kv_heads) * blocks * waves <= kSufResidentWaves ? kSufPaired : kSufLongFirst;
     const uint64_t groups = static_cast<uint64_t>(view->kv_heads) * plan.splits;
     const uint64_t wgs = (groups * blocks + 7) / 8 * 8;
     if (wgs > 0x7fffffffu) return MIIKV_EINVAL;
     const dim3 grid(static_cast<uint32_t>(wgs));
-    if (view->head_dim == 128) hipLaunchKernelGGL(suffix_kernel<128>, grid, dim3(64 * kSufWaves), 0, s, a);
-    else hipLaunchKernelGGL(suffix_kernel<256>, grid, dim3(64 * kSufWaves), 0, s, a);
+    const dim3 block(64 * waves);
+    if (waves == kSufWaves) {
+        if (view->head_dim == 128) hipLaunchKernelGGL((suffix_kernel<128, kSufWaves>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((suffix_kernel<256, kSufWaves>), grid, block, 0, s, a);
+    } else {
+        if (view->head_dim == 128) hipLaunchKernelGGL((suffix_kernel<128, kSufWavesSmall>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((suffix_kernel<256, kSufWavesSmall>), grid, block, 0, s, a);
+    }
     if (plan.splits > 1) launch_suffix_combine(view, q_heads, G, token_count, base_position, prefill_state, plan,
                                                a.part, out, gate, gated_out, s);
     return hip_status(hipGetLastError());

@@ -5,18 +5,19 @@
 
 namespace miikv {
 
-#ifndef MIIKV_SUFFIX_WAVES
-#define MIIKV_SUFFIX_WAVES 8
-#endif
-constexpr uint32_t kSufWaves = MIIKV_SUFFIX_WAVES;
-constexpr uint32_t kSufRows = 32 * kSufWaves;  // query rows per workgroup
+// suffix_kernel's two forms: 8 waves (256 query rows) per workgroup, one workgroup per CU,
+// and 4 waves (128 rows) with half the LDS, two workgroups per CU.
+constexpr uint32_t kSufWaves = 8;
+constexpr uint32_t kSufWavesSmall = 4;
 constexpr uint32_t kSufStep = 32;              // keys per step
 constexpr float kLog2eS = 1.4426950408889634f;
 constexpr float kSlackS = 6.0f;        // lazy-rescale threshold (log2 units): p <= 64
-// Resident workgroups of suffix_kernel on the chip: 256 CUs, each holding 8 waves
-// (two per SIMD at <= 256 VGPRs) and its LDS tile buffers (4 x 32 KiB at D = 256).
-constexpr uint32_t kSufSlots = 256 * (8 / kSufWaves);
+// Resident waves of suffix_kernel on the chip: 256 CUs, two waves per SIMD (at <= 256
+// VGPRs), in LDS tile buffers of 128 KiB per CU at D = 256.
+constexpr uint32_t kSufResidentWaves = 256 * 8;
 constexpr uint32_t kSufMaxSplits = 64;
+constexpr uint32_t kSufMinKeys = 256;  // keys per split, at least: 8-wave form
+constexpr uint32_t kSufMinKeysSmall = 160;  // 4-wave form
 // Suffixes of at most this many decode row sets (tokens / tokens packed per row set)
 // run as a batch of decodes (miikv_decode.hip): caches of more than 16384 positions,
 // and of at most that many.
@@ -56,6 +57,13 @@ struct ExpandArgs {
     uint32_t current;
 };
 
+// Order of (kv head, split, row block) along an XCD's workgroups: the row blocks of one
+// (kv head, split) next to each other; the splits of one row block next to each other; or,
+// without splits, each kv head's row blocks with the most keys first (kSufLongFirst), in
+// the 4-wave form the second half shortest first (kSufPaired): the two workgroups that a
+// CU then runs together have about the same keys in all.
+enum SuffixOrder : uint32_t { kSufTilesTogether = 0, kSufRowsTogether = 1, kSufLongFirst = 2, kSufPaired = 3 };
+
 struct SuffixArgs {
     Geo g;
     const void* q;
@@ -75,7 +83,7 @@ struct SuffixArgs {
     float* out;
     const float* gate;
     float* gated_out;
-    uint32_t rows_together;  // suffix_kernel order: (kv head, row block, split) when set
+    uint32_t order;        // suffix_kernel order of the work items (SuffixOrder)
 };
 
 // Partial records of split-K, laid out so that a wave's 32 rows write one
@@ -116,6 +124,23 @@ template <uint32_t N>
 __device__ __forceinline__ void wait_vmem_le() {
     static_assert(N < 64, "vmcnt holds 6 bits");
     asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
+}
+
+// 16 bytes per lane from `src` (per lane) to LDS at `lds` + 16 * lane (`lds` wave-uniform).
+// In asm: the compiler drains every load that it knows of at a barrier, these copies too;
+// here the caller counts them (wait_vmem_le).
+__device__ __forceinline__ void copy_to_lds(const void* src, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                 :
+                 : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(src)
+                 : "memory", "m0");
+}
+__device__ __forceinline__ uint32_t lds_offset(const void* p) {
+    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void*)p));
+}
+// Workgroup barrier after this wave's LDS reads have returned; copies stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
 }  // namespace miikv

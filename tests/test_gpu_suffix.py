@@ -715,3 +715,29 @@ def test_suffix_random(gpu, seed):
     assert_attention_close(out.cpu().numpy(), expect, what)
     if gate is not None:
         assert_attention_close(gated.cpu().numpy(), expect / (1 + np.exp(-gate)), what + " gated")
+
+
+@pytest.mark.parametrize("hq,hk,d,prefix,t", [
+    (32, 8, 128, 0, 1100),   # 4 waves, unsplit, odd number of row blocks paired per CU
+    (24, 4, 256, 0, 1403),   # the same, even
+    (24, 4, 256, 0, 77),     # 4 waves, one workgroup per CU, last row block partial
+    (24, 4, 256, 700, 33),   # 4 waves, split, fewer rows than two row blocks
+    (32, 8, 128, 159, 129),  # 4 waves, key ranges of unequal length
+    (32, 8, 128, 5, 2100),   # 8 waves, more workgroups than fit at once, longest first
+])
+def test_suffix_workgroup_forms(gpu, hq, hk, d, prefix, t):
+    """Both forms of the MFMA kernel and each order of its work items, with row blocks and
+    key ranges that end inside one, against attention in float64 over the dequantised cache."""
+    import miinfer_amd as m
+    rng = np.random.default_rng(prefix + t)
+    n = prefix + t
+    cache = m.KvCache.contiguous(hk, d, (n + 63) // 64 * 64)
+    cache.append(_dev(randn_f16(rng, (n, hk, d)), gpu), _dev(randn_f16(rng, (n, hk, d)), gpu))
+    q = _dev(randn_f16(rng, (t, hq, d)), gpu)
+    out, _ = m.suffix_attention(cache, q, prefix)
+    k, v = (x.double() for x in cache.export_dequant(0, 0, n))
+    hidden = torch.arange(n, device=gpu)[None, :] > prefix + torch.arange(t, device=gpu)[:, None]
+    for h in range(hq):
+        s = q[:, h].double() @ k[h // (hq // hk)].T.contiguous() / math.sqrt(d)
+        expect = torch.softmax(s.masked_fill(hidden, -math.inf), -1) @ v[h // (hq // hk)]
+        assert_attention_close(out[:, h].cpu().numpy(), expect.cpu().numpy(), f"head {h}")
