@@ -57,18 +57,39 @@ __device__ __forceinline__ uint32_t context_keys(uint32_t host_count, const miik
     return ps ? min(host_count, ps->base_position + ps->token_count) : host_count;
 }
 
+// Sixteen signed codes as packed bytes.
+__device__ __forceinline__ uint4 pack16_codes(const int8_t (&q)[16]) {
+    uint32_t w[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+        w[u] = static_cast<uint32_t>(static_cast<uint8_t>(q[4 * u])) |
+               (static_cast<uint32_t>(static_cast<uint8_t>(q[4 * u + 1])) << 8) |
+               (static_cast<uint32_t>(static_cast<uint8_t>(q[4 * u + 2])) << 16) |
+               (static_cast<uint32_t>(static_cast<uint8_t>(q[4 * u + 3])) << 24);
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
 // One 32-key step of kv head blockIdx.y: 256 threads; keys at or past the context
 // end become 0 (their codes may never have been written).
-// Fused append (APPEND, a.k_new set): a step holding any of the suffix's own keys
-// [P, P + T) first assembles its 32-token group in LDS -- the cached codes and
-// scales of the other keys, the suffix rows quantised with the append rule (the
-// bytes miikv_append_f16 stores) -- writes the whole group back to the cache with
-// 16-byte stores and expands it from LDS.
+// Bound: the latency of one chain (block table, codes and scales, tiles) in short
+// contexts, HBM in long ones.  So a thread issues every read of the step at once: K codes
+// as whole 16-byte words of the cache tile (one key, 8 dims of two blocks: one piece of
+// two fragments, both scales in one word), V codes as one dim's keys (all fragments of the
+// dim's lane).
+// Fused append (APPEND, a.k_new set): in a step holding any of the suffix's own keys
+// [P, P + T) those are quantised with the append rule (the bytes miikv_append_f16 stores)
+// into LDS, K in the cache's order, V row by row (a thread then gathers its dim's bytes
+// without bank conflicts); the same registers go to the cache and into the tiles.
+// Against 8- and 4-byte reads per fragment piece and byte stores of V into the cache's
+// order: 24q/4kv/D256, 77 tokens fused over 3001 paged, 9.6 -> 7.2 us of 38.8 -> 36.3 a
+// layer; config 4 fused 12.9 -> 10.5 us (53 MB, 5.0 TB/s).
 template <uint32_t D, bool APPEND>
 __global__ void __launch_bounds__(256) expand_kernel(ExpandArgs a) {
     constexpr uint32_t NB = D / 32;
-    constexpr uint32_t NKF = D / 16;       // K fragments per step
-    constexpr uint32_t PER = D / 64;       // fragment lanes per thread, per operand
+    constexpr uint32_t NKF = D / 16;             // K fragments per step
+    constexpr uint32_t KW = kSufStep * D / 4096;  // K words per thread
+    constexpr uint32_t DT = 256 / D;             // threads per dim (V)
+    constexpr uint32_t VG = 4 / DT;              // 8-key groups G of the dim per thread
     __shared__ __align__(16) _Float16 s_vs[NB * kSufStep];  // [block][key]
     __shared__ __align__(16) uint8_t s_grp[APPEND ? 2 * kSufStep * D + 2 * kSufStep * NB * 2 : 16];
     const Geo& geo = a.g;
@@ -81,59 +102,80 @@ __global__ void __launch_bounds__(256) expand_kernel(ExpandArgs a) {
     const uint32_t tok0 = step * kSufStep;
     if (tok0 >= nkeys) return;
     if (a.current && a.ps != nullptr && step < a.ps->base_position / kSufStep) return;  // already expanded
-    const size_t slab = slab_of(geo, a.seq, tok0, h);
-    const uint32_t tp0 = tok0 % geo.page_tokens;
-    const size_t sc0 = (slab * geo.page_tokens + tp0) * NB;
-    const size_t cb = slab * static_cast<size_t>(geo.page_tokens) * D + static_cast<size_t>(tp0) * D;
-    const int8_t* kb = geo.k_codes + cb;
-    const int8_t* vb = geo.v_codes + cb;
-    // fp16 planes (the control path): the tiles are the stored fp16 rows themselves
-    const _Float16* kb16 = reinterpret_cast<const _Float16*>(geo.k_codes) + cb;
-    const _Float16* vb16 = reinterpret_cast<const _Float16*>(geo.v_codes) + cb;
-    const uint16_t* ksc = geo.k_scales + sc0;
-    const uint16_t* vsc = geo.v_scales + sc0;
+    // The suffix's own keys in this step: [own_lo, own_hi), none without the fused append.
+    uint32_t own_lo = 0, own_hi = 0;
     if constexpr (APPEND) {
         const uint32_t P = a.ps ? a.ps->base_position : a.base_position;
         const uint32_t T = a.ps ? min(a.token_count, a.ps->token_count) : a.token_count;
-        if (tok0 + kSufStep > P && tok0 < P + T) {
-            // The suffix rows of this step, thread (key tl, 16-dim chunk q16) per item,
-            // loaded first so that they travel with the cached group below.
-            constexpr uint32_t ITEMS = kSufStep * (D / 16) / 256;
-            uint4 rk[ITEMS][2], rv[ITEMS][2];
+        own_lo = min(max(P, tok0) - tok0, kSufStep);
+        own_hi = min(max(P + T, tok0) - tok0, kSufStep);
+    }
+    const bool owned = APPEND && own_lo < own_hi;
+    auto own = [&](uint32_t key) { return APPEND && key >= own_lo && key < own_hi; };
+    // Its rows go out ahead of the block table's round trip.  Thread (key tl, 16-dim chunk
+    // q16) per item; partner lanes q16 ^ 1 hold the two halves of a 32-value block.
+    constexpr uint32_t ITEMS = APPEND ? kSufStep * (D / 16) / 256 : 1;
+    uint4 rk[ITEMS][2], rv[ITEMS][2];
+    if constexpr (APPEND) {
+        if (owned) {
+            const uint32_t P = a.ps ? a.ps->base_position : a.base_position;
 #pragma unroll
             for (uint32_t it = 0; it < ITEMS; ++it) {
                 const uint32_t w = tid + 256 * it, tl = w / (D / 16), q16 = w % (D / 16);
-                const uint32_t key = tok0 + tl;
-                const uint32_t t = key >= P && key < P + T ? key - P : 0;
+                const uint32_t t = own(tl) ? tok0 + tl - P : 0;
                 const size_t src = (static_cast<size_t>(t) * geo.kv_heads + h) * D + q16 * 16;
                 rk[it][0] = *reinterpret_cast<const uint4*>(a.k_new + src);
                 rk[it][1] = *reinterpret_cast<const uint4*>(a.k_new + src + 8);
                 rv[it][0] = *reinterpret_cast<const uint4*>(a.v_new + src);
                 rv[it][1] = *reinterpret_cast<const uint4*>(a.v_new + src + 8);
             }
-            // Group in LDS: [K codes 32*D][V codes 32*D][K scales 32*NB][V scales 32*NB]
-            // in the cache's slab order.  Copy the cached group (its keys outside the
-            // suffix keep their bytes), then overwrite the suffix keys.
-            uint4* g16 = reinterpret_cast<uint4*>(s_grp);
-            constexpr uint32_t CK = kSufStep * D / 16, CS = kSufStep * NB * 2 / 16;
-            for (uint32_t c = tid; c < 2 * CK + 2 * CS; c += 256) {
-                const uint4* src = c < CK ? reinterpret_cast<const uint4*>(kb) + c
-                                 : c < 2 * CK ? reinterpret_cast<const uint4*>(vb) + (c - CK)
-                                 : c < 2 * CK + CS ? reinterpret_cast<const uint4*>(ksc) + (c - 2 * CK)
-                                                   : reinterpret_cast<const uint4*>(vsc) + (c - 2 * CK - CS);
-                g16[c] = *src;
+        }
+    }
+    const size_t slab = slab_of(geo, a.seq, tok0, h);
+    const uint32_t tp0 = tok0 % geo.page_tokens;
+    const size_t sc0 = (slab * geo.page_tokens + tp0) * NB;
+    const size_t cb = slab * static_cast<size_t>(geo.page_tokens) * D + static_cast<size_t>(tp0) * D;
+    const uint16_t* ksc = geo.k_scales + sc0;
+    const uint16_t* vsc = geo.v_scales + sc0;
+    _Float16* out = a.tiles + (static_cast<size_t>(h) * a.steps + step) * tile_halves(D);
+    // K word w = tid + 256u of the cache group: key 16(w / D) + w % 16, dims 64cc + 8g .. and
+    // 64cc + 32 + 8g .., cc = (w % D) / 64, g = (w / 16) % 4; fragment c, lane (n, hh) holds
+    // key n, dims 16c + 8hh .. +7.
+    uint4 kw[KW];
+    uint32_t ks2[KW];
+    // V dim vd, groups G = vg0, vg0 + DT, ..: word x (y) of a group holds keys 4G .. +3 (16 +
+    // 4G .. +3); fragment f = 2mt + kc, lane (n, hh) holds dim 32mt + n, keys 16kc + 4hh .. +3
+    // and 16kc + 8 + 4hh .. +3 (G = hh and 2 + hh).
+    const uint32_t vd = tid % D, vg0 = tid / D;
+    uint2 vw[VG];
+    if (!geo.v_f16 && tid < kSufStep * NB) {  // V scales to [block][key]; the suffix's own keys below
+        const uint32_t key = tid / NB, blk = tid % NB;
+        if (!own(key)) s_vs[blk * kSufStep + key] = tok0 + key < nkeys ? clamp_scale(vsc[tid]) : (_Float16)0.0f;
+    }
+    if (!geo.k_f16) {
+#pragma unroll
+        for (uint32_t u = 0; u < KW; ++u) {
+            const uint32_t w = tid + 256 * u, key = 16 * (w / D) + w % 16, cc = (w % D) / 64;
+            if (!own(key)) {
+                ks2[u] = *reinterpret_cast<const uint32_t*>(ksc + key * NB + 2 * cc);
+                kw[u] = *reinterpret_cast<const uint4*>(geo.k_codes + cb + 16 * static_cast<size_t>(w));
             }
-            __syncthreads();
+        }
+    }
+    if (!geo.v_f16 && !(owned && own_lo == 0 && own_hi == kSufStep)) {
+#pragma unroll
+        for (uint32_t x = 0; x < VG; ++x)
+            vw[x] = *reinterpret_cast<const uint2*>(geo.v_codes + cb + vd * 32 + 8 * (vg0 + DT * x));
+    }
+    if constexpr (APPEND) {
+        if (owned) {
             uint8_t* s_k = s_grp;
             uint8_t* s_v = s_grp + kSufStep * D;
-            uint16_t* s_ks = reinterpret_cast<uint16_t*>(s_grp + 2 * kSufStep * D);
+            uint16_t* s_ks = reinterpret_cast<uint16_t*>(s_grp + 2 * kSufStep * D);  // [key][block]
             uint16_t* s_vsc = s_ks + kSufStep * NB;
-            // partner lanes q16 ^ 1 hold the two halves of a 32-value block
 #pragma unroll
             for (uint32_t it = 0; it < ITEMS; ++it) {
-                const uint32_t w = tid + 256 * it, tl = w / (D / 16), q16 = w % (D / 16);
-                const uint32_t key = tok0 + tl;
-                const bool mine = key >= P && key < P + T;
+                const uint32_t w = tid + 256 * it, tl = w / (D / 16), q16 = w % (D / 16), d0 = 16 * q16;
                 float xk[16], xv[16];
                 unpack16_f16(rk[it], xk);
                 unpack16_f16(rv[it], xv);
@@ -141,72 +183,85 @@ __global__ void __launch_bounds__(256) expand_kernel(ExpandArgs a) {
                 float sk, sv;
                 quantize16(xk, qk, sk);  // both lanes of a pair reach the shuffles
                 quantize16(xv, qv, sv);
-                if (!mine) continue;
-                const uint32_t d0 = q16 * 16;
-                uint32_t packed[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    packed[u] = static_cast<uint32_t>(static_cast<uint8_t>(qk[4 * u])) |
-                                (static_cast<uint32_t>(static_cast<uint8_t>(qk[4 * u + 1])) << 8) |
-                                (static_cast<uint32_t>(static_cast<uint8_t>(qk[4 * u + 2])) << 16) |
-                                (static_cast<uint32_t>(static_cast<uint8_t>(qk[4 * u + 3])) << 24);
-                *reinterpret_cast<uint2*>(s_k + k_code_offset(tl, d0, D)) = make_uint2(packed[0], packed[1]);
-                *reinterpret_cast<uint2*>(s_k + k_code_offset(tl, d0 + 8, D)) = make_uint2(packed[2], packed[3]);
-#pragma unroll
-                for (int u = 0; u < 16; ++u) s_v[v_code_offset(tl, d0 + u, D)] = static_cast<uint8_t>(qv[u]);
+                if (!own(tl)) continue;
+                const uint4 pk = pack16_codes(qk);
+                *reinterpret_cast<uint2*>(s_k + k_code_offset(tl, d0, D)) = make_uint2(pk.x, pk.y);
+                *reinterpret_cast<uint2*>(s_k + k_code_offset(tl, d0 + 8, D)) = make_uint2(pk.z, pk.w);
+                *reinterpret_cast<uint4*>(s_v + tl * D + d0) = pack16_codes(qv);
                 if ((q16 & 1) == 0) {
+                    const uint16_t vbits = f32_to_f16_bits(sv);
                     s_ks[tl * NB + d0 / 32] = f32_to_f16_bits(sk);
-                    s_vsc[tl * NB + d0 / 32] = f32_to_f16_bits(sv);
+                    s_vsc[tl * NB + d0 / 32] = vbits;
+                    s_vs[(d0 / 32) * kSufStep + tl] = clamp_scale(vbits);  // its own keys are context keys
                 }
             }
             __syncthreads();
-            for (uint32_t c = tid; c < 2 * CK + 2 * CS; c += 256) {
-                uint4* dst = c < CK ? reinterpret_cast<uint4*>(geo.k_codes + cb) + c
-                           : c < 2 * CK ? reinterpret_cast<uint4*>(geo.v_codes + cb) + (c - CK)
-                           : c < 2 * CK + CS ? reinterpret_cast<uint4*>(geo.k_scales + sc0) + (c - 2 * CK)
-                                             : reinterpret_cast<uint4*>(geo.v_scales + sc0) + (c - 2 * CK - CS);
-                *dst = g16[c];
+            int8_t* kdst = geo.k_codes + cb;
+#pragma unroll
+            for (uint32_t u = 0; u < KW; ++u) {
+                const uint32_t w = tid + 256 * u, key = 16 * (w / D) + w % 16, cc = (w % D) / 64;
+                if (!own(key)) continue;
+                ks2[u] = *reinterpret_cast<const uint32_t*>(s_ks + key * NB + 2 * cc);
+                kw[u] = *reinterpret_cast<const uint4*>(s_k + 16 * w);
+                *reinterpret_cast<uint4*>(kdst + 16 * static_cast<size_t>(w)) = kw[u];
             }
-            kb = reinterpret_cast<const int8_t*>(s_k);
-            vb = reinterpret_cast<const int8_t*>(s_v);
-            ksc = s_ks;
-            vsc = s_vsc;
+#pragma unroll
+            for (uint32_t x = 0; x < VG; ++x) {
+                const uint32_t g = vg0 + DT * x;
+                uint32_t word[2] = {vw[x].x, vw[x].y};
+#pragma unroll
+                for (uint32_t J = 0; J < 2; ++J) {
+                    uint32_t own_word = 0, mask = 0;
+#pragma unroll
+                    for (uint32_t I = 0; I < 4; ++I) {
+                        const uint32_t key = 16 * J + 4 * g + I;
+                        own_word |= static_cast<uint32_t>(s_v[key * D + vd]) << (8 * I);
+                        if (own(key)) mask |= 0xffu << (8 * I);
+                    }
+                    word[J] = (word[J] & ~mask) | (own_word & mask);
+                }
+                vw[x] = make_uint2(word[0], word[1]);
+                *reinterpret_cast<uint2*>(geo.v_codes + cb + vd * 32 + 8 * g) = vw[x];
+            }
+            if (tid < kSufStep * NB && own(tid / NB)) {
+                geo.k_scales[sc0 + tid] = s_ks[tid];
+                geo.v_scales[sc0 + tid] = s_vsc[tid];
+            }
         }
     }
-    if (tid < kSufStep * NB && !geo.v_f16) {
-        const uint32_t key = tid / NB, blk = tid % NB;
-        s_vs[blk * kSufStep + key] = tok0 + key < nkeys ? clamp_scale(vsc[tid]) : (_Float16)0.0f;
-    }
-    __syncthreads();
-    _Float16* out = a.tiles + (static_cast<size_t>(h) * a.steps + step) * tile_halves(D);
-    // K fragment c, lane (n, hh): key n, dims 16c + 8hh .. +7.  In the cache tile
-    // those 8 codes sit at (key/16)*16D + (c/4)*1024 + g*256 + (key%16)*16 + e*8
-    // with e = (c%4)/2, g = 2*(c%2) + hh.
+    if (!owned) __syncthreads();  // s_vs
+
+    if (geo.k_f16) {
+        // fp16 planes (the control path): the tiles are the stored fp16 rows themselves,
+        // fragment c's 8 halves at the offset of the codes
+        const _Float16* kb16 = reinterpret_cast<const _Float16*>(geo.k_codes) + cb;
 #pragma unroll
-    for (uint32_t u = 0; u < PER; ++u) {
-        const uint32_t fl = tid + 256 * u;
-        const uint32_t c = fl / 64, l = fl % 64, n = l % 32, hh = l / 32;
-        const uint32_t off = (n / 16) * 16 * D + (c / 4) * 1024 + (2 * (c % 2) + hh) * 256 + (n % 16) * 16 +
-                             ((c % 4) / 2) * 8;
-        if (geo.k_f16) {
-            const half8 x = *reinterpret_cast<const half8*>(kb16 + off);
+        for (uint32_t u = 0; u < D / 64; ++u) {
+            const uint32_t fl = tid + 256 * u;
+            const uint32_t c = fl / 64, l = fl % 64, n = l % 32, hh = l / 32;
+            const half8 x = *reinterpret_cast<const half8*>(kb16 + k_code_offset(n, 16 * c + 8 * hh, D));
             *reinterpret_cast<half8*>(out + 8 * fl) = tok0 + n < nkeys ? x : half8{};
-            continue;
         }
-        const uint2 w = *reinterpret_cast<const uint2*>(kb + off);
-        const _Float16 sc = tok0 + n < nkeys ? clamp_scale(ksc[n * NB + c / 2]) : (_Float16)0.0f;
-        *reinterpret_cast<half8*>(out + 8 * fl) = codes8_to_half8(w.x, w.y) * (half8)sc;
-    }
-    // V fragment f = 2mt + kc, lane (n, hh): dim 32mt + n, positions 4*b3 + i hold
-    // keys 16kc + 8*b3 + 4hh + i.  A 32-token group stores dim d's code of key
-    // 16J + 4G + I at d*32 + 8G + 4J + I, so b3 = 0 is the dword at G = hh and
-    // b3 = 1 the dword at G = 2 + hh, both at J = kc.
+    } else {
 #pragma unroll
-    for (uint32_t u = 0; u < PER; ++u) {
-        const uint32_t fl = tid + 256 * u;
-        const uint32_t f = fl / 64, l = fl % 64, n = l % 32, hh = l / 32;
-        const uint32_t mt = f / 2, kc = f % 2;
-        if (geo.v_f16) {
+        for (uint32_t u = 0; u < KW; ++u) {
+            const uint32_t w = tid + 256 * u, n = 16 * (w / D) + w % 16, cc = (w % D) / 64, g = (w / 16) % 4;
+            const bool live = tok0 + n < nkeys;
+            const _Float16 lo = live ? clamp_scale(static_cast<uint16_t>(ks2[u])) : (_Float16)0.0f;
+            const _Float16 hi = live ? clamp_scale(static_cast<uint16_t>(ks2[u] >> 16)) : (_Float16)0.0f;
+            _Float16* o = out + 8 * ((4 * cc + g / 2) * 64 + (g % 2) * 32 + n);
+            *reinterpret_cast<half8*>(o) = codes8_to_half8(kw[u].x, kw[u].y) * (half8)lo;
+            *reinterpret_cast<half8*>(o + 2 * 64 * 8) = codes8_to_half8(kw[u].z, kw[u].w) * (half8)hi;
+        }
+    }
+    _Float16* vout = out + 64 * 8 * NKF;
+    if (geo.v_f16) {
+        const _Float16* vb16 = reinterpret_cast<const _Float16*>(geo.v_codes) + cb;
+#pragma unroll
+        for (uint32_t u = 0; u < D / 64; ++u) {
+            const uint32_t fl = tid + 256 * u;
+            const uint32_t f = fl / 64, l = fl % 64, n = l % 32, hh = l / 32;
+            const uint32_t mt = f / 2, kc = f % 2;
             const _Float16* vd16 = vb16 + (32 * mt + n) * 32;
             half4 a0 = *reinterpret_cast<const half4*>(vd16 + 8 * hh + 4 * kc);
             half4 a1 = *reinterpret_cast<const half4*>(vd16 + 8 * (2 + hh) + 4 * kc);
@@ -218,19 +273,24 @@ __global__ void __launch_bounds__(256) expand_kernel(ExpandArgs a) {
             half8 r;
             r.lo = a0;
             r.hi = a1;
-            *reinterpret_cast<half8*>(out + 64 * 8 * NKF + 8 * fl) = r;
-            continue;
+            *reinterpret_cast<half8*>(vout + 8 * fl) = r;
         }
-        const int8_t* vd = vb + (32 * mt + n) * 32;
-        const uint32_t w0 = *reinterpret_cast<const uint32_t*>(vd + 8 * hh + 4 * kc);
-        const uint32_t w1 = *reinterpret_cast<const uint32_t*>(vd + 8 * (2 + hh) + 4 * kc);
-        const _Float16* sv = &s_vs[mt * kSufStep + 16 * kc + 4 * hh];
-        const half4 a0 = codes4_to_half4(w0) * *reinterpret_cast<const half4*>(sv);
-        const half4 a1 = codes4_to_half4(w1) * *reinterpret_cast<const half4*>(sv + 8);
-        half8 r;
-        r.lo = a0;
-        r.hi = a1;
-        *reinterpret_cast<half8*>(out + 64 * 8 * NKF + 8 * fl) = r;
+    } else {
+        const uint32_t mt = vd / 32, n = vd % 32;
+#pragma unroll
+        for (uint32_t x = 0; x < VG / 2; ++x) {  // hh = vg0 + DT * x: groups x and x + VG / 2
+            const uint32_t hh = vg0 + DT * x;
+#pragma unroll
+            for (uint32_t kc = 0; kc < 2; ++kc) {
+                const uint32_t w0 = kc == 0 ? vw[x].x : vw[x].y;
+                const uint32_t w1 = kc == 0 ? vw[x + VG / 2].x : vw[x + VG / 2].y;
+                const _Float16* sv = &s_vs[mt * kSufStep + 16 * kc + 4 * hh];
+                half8 r;
+                r.lo = codes4_to_half4(w0) * *reinterpret_cast<const half4*>(sv);
+                r.hi = codes4_to_half4(w1) * *reinterpret_cast<const half4*>(sv + 8);
+                *reinterpret_cast<half8*>(vout + 8 * ((2 * mt + kc) * 64 + hh * 32 + n)) = r;
+            }
+        }
     }
 }
 
