@@ -3,6 +3,7 @@
 
 #include <cmath>
 #include <cstdlib>
+#include <type_traits>
 
 namespace miikv {
 
@@ -55,10 +56,18 @@ __device__ __forceinline__ void load16_f32(const float* p, float (&x)[16]) {
     }
 }
 
-// K prologue on one lane's 16 dims d0 = 16*q16 ..: RMSNorm * weight, then RoPE on
-// dims 0..63 (gfx906/kernels/qwen3_primitives.hip:7257-7281, 622-659).
+// Value of lane ^ 4 (DPP row shifts by 4 towards each other, one per pair of quads).
+__device__ __forceinline__ float dpp_xor4(float x) {
+    const int v = __builtin_bit_cast(int, x);
+    const int up = __builtin_amdgcn_update_dpp(v, v, 0x104, 0xF, 0x5, false);   // row_shl:4, quads 0 and 2
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(up, v, 0x114, 0xF, 0xA, false));  // row_shr:4, 1 and 3
+}
+
+// K prologue on one lane's 16 dims d0 = 16*q16 .. of a row held by GROUPS = D/16
+// consecutive lanes: RMSNorm * weight, then RoPE on dims 0..63
+// (gfx906/kernels/qwen3_primitives.hip:7257-7281, 622-659).
 // The sum of squares follows the reference's 256-lane LDS tree exactly: element t
-// first meets t + D/2 (lanes q16 and q16 ^ groups/2), then t + D/4, ... down to the
+// first meets t + D/2 (lanes q16 and q16 ^ GROUPS/2), then t + D/4, ... down to the
 // lane's own 16 values, pairs 8, 4, 2, 1 apart.  r = 1 / sqrt(ss / D + eps) with the
 // correctly rounded square root and division (the reference's rsqrtf is the
 // hardware approximation, within one ulp of it), value * r * weight in that order.
@@ -68,21 +77,27 @@ __device__ __forceinline__ void load16_f32(const float* p, float (&x)[16]) {
 // kernel, so the angles are the ones a host computes), and rotated with rope_sincos
 // (the reference calls cosf and sinf).  No contraction into fused multiply-adds: every
 // product and sum rounds as written, as in the oracle.
-__device__ __forceinline__ void k_norm_rope16(float (&x)[16], const float* w, uint32_t q16, uint32_t groups,
-                                              uint32_t D, uint32_t position, float step, float eps) {
+// The tree's levels across lanes are DPP moves.  `rotation`(j) gives the sine and cosine of
+// pair 16 * (q16 & 1) + j, asked in order by the lanes q16 < 4.
+template <uint32_t GROUPS, typename F>
+__device__ __forceinline__ void k_norm_rope16(float (&x)[16], const float* w, uint32_t q16, float eps, F rotation) {
 #pragma clang fp contract(off)
+    static_assert(GROUPS == 8 || GROUPS == 16, "D = 128 or 256");
     float sq[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) sq[i] = x[i] * x[i];
-    for (uint32_t o = groups / 2; o > 0; o >>= 1) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) sq[i] += __shfl_xor(sq[i], o, 64);
+    for (int i = 0; i < 16; ++i) {
+        if constexpr (GROUPS == 16) sq[i] += dpp_mov<0x128>(sq[i]);  // row_ror:8: lane ^ 8
+        sq[i] += dpp_xor4(sq[i]);
+        sq[i] += dpp_mov<0x4E>(sq[i]);  // lane ^ 2
+        sq[i] += dpp_mov<0xB1>(sq[i]);  // lane ^ 1
     }
 #pragma unroll
     for (int s2 = 8; s2 > 0; s2 >>= 1)
 #pragma unroll
         for (int i = 0; i < s2; ++i) sq[i] += sq[i + s2];
-    const float r = 1.0f / sqrtf(sq[0] / static_cast<float>(D) + eps);
+    const float r = 1.0f / sqrtf(sq[0] / static_cast<float>(16 * GROUPS) + eps);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const float4 wv = *reinterpret_cast<const float4*>(w + 16 * q16 + 4 * i);
@@ -91,26 +106,28 @@ __device__ __forceinline__ void k_norm_rope16(float (&x)[16], const float* w, ui
         x[4 * i + 2] = x[4 * i + 2] * r * wv.z;
         x[4 * i + 3] = x[4 * i + 3] * r * wv.w;
     }
-    float partner[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) partner[i] = dpp_mov<0x4E>(x[i]);  // lane ^ 2
     if (q16 >= 4) return;
-    float angle = static_cast<float>(position);
-    // first pair index of this lane: 0, or 16 (step applied 16 times, in order)
-#pragma unroll
-    for (uint32_t i = 0; i < 16; ++i) {
-        const float next = angle * step;
-        angle = (q16 & 1) ? next : angle;
-    }
-    const bool low = q16 < 2;           // dims i (low) or i + 32 (high) of the pairs
+    const bool low = q16 < 2;  // dims i (low) or i + 32 (high) of the pairs
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
-        float sn, cs;
-        rope_sincos(angle, &sn, &cs);
-        if (low) x[j] = x[j] * cs - partner[j] * sn;
-        else x[j] = partner[j] * sn + x[j] * cs;
-        angle *= step;
+        const float partner = dpp_mov<0x4E>(x[j]);  // lane ^ 2
+        const float2 sc = rotation(j);
+        x[j] = low ? x[j] * sc.y - partner * sc.x : partner * sc.x + x[j] * sc.y;
     }
+}
+
+// The angle of pair i: position * step * step ... (i factors, in that order).  Unrolled
+// with selects: the factors that count differ per lane.
+template <uint32_t MOST>
+__device__ __forceinline__ float rope_angle(uint32_t position, float step, uint32_t i) {
+#pragma clang fp contract(off)
+    float angle = static_cast<float>(position);
+#pragma unroll
+    for (uint32_t k = 0; k < MOST; ++k) {
+        const float next = angle * step;
+        angle = k < i ? next : angle;
+    }
+    return angle;
 }
 
 // Eight values -> eight fp16 (round to nearest even) in one 16-byte word.
@@ -120,6 +137,36 @@ __device__ __forceinline__ uint4 pack8_f16(const float* x) {
     for (int i = 0; i < 4; ++i)
         w[i] = static_cast<uint32_t>(f32_to_f16_bits(x[2 * i])) | (static_cast<uint32_t>(f32_to_f16_bits(x[2 * i + 1])) << 16);
     return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// One lane's 16 dims of a K and a V row of q8 codes to token tp of the slab: K as runs of
+// 8 in the tiled layout, V an element per dim.
+__device__ __forceinline__ void store_k_codes16(const Geo& g, size_t slab, uint32_t tp, uint32_t q16, uint4 k, float sk) {
+    const uint32_t D = g.head_dim, d0 = 16 * q16;
+    int8_t* kslab = g.k_codes + slab * static_cast<size_t>(g.page_tokens) * D;
+    *reinterpret_cast<uint2*>(kslab + k_code_offset(tp, d0, D)) = make_uint2(k.x, k.y);
+    *reinterpret_cast<uint2*>(kslab + k_code_offset(tp, d0 + 8, D)) = make_uint2(k.z, k.w);
+    if ((q16 & 1) == 0) g.k_scales[(slab * g.page_tokens + tp) * (D / 32) + d0 / 32] = f32_to_f16_bits(sk);
+}
+__device__ __forceinline__ void store_v_codes16(const Geo& g, size_t slab, uint32_t tp, uint32_t q16, uint4 v, float sv) {
+    const uint32_t D = g.head_dim, d0 = 16 * q16;
+    int8_t* vslab = g.v_codes + slab * static_cast<size_t>(g.page_tokens) * D;
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 16; ++i) vslab[v_code_offset(tp, d0 + i, D)] = static_cast<int8_t>(w[i / 4] >> (8 * (i % 4)));
+    if ((q16 & 1) == 0) g.v_scales[(slab * g.page_tokens + tp) * (D / 32) + d0 / 32] = f32_to_f16_bits(sv);
+}
+
+// The prologue with each rotating lane computing its own 16 sines and cosines.
+template <uint32_t GROUPS>
+__device__ __forceinline__ void k_prologue16(const AppendIn& in, float (&x)[16], uint32_t q16, uint32_t pos) {
+    float angle = rope_angle<16>(pos, in.rope_step, 16 * (q16 & 1));
+    k_norm_rope16<GROUPS>(x, in.k_norm_weight, q16, in.epsilon, [&](int) __attribute__((always_inline)) {
+        float2 sc;
+        rope_sincos(angle, &sc.x, &sc.y);
+        angle *= in.rope_step;
+        return sc;
+    });
 }
 
 // One thread per (row, 16-dim group); a row is (token, kv_head).  Adjacent
@@ -164,7 +211,7 @@ __global__ void __launch_bounds__(256) append_kernel(
         load16_f32(static_cast<const float*>(in.k) + src, xk);
         load16_f32(static_cast<const float*>(in.v) + src, xv);
         if (in.k_norm_weight != nullptr)
-            k_norm_rope16(xk, in.k_norm_weight, q16, groups, D, pos, in.rope_step, in.epsilon);
+            groups == 16 ? k_prologue16<16>(in, xk, q16, pos) : k_prologue16<8>(in, xk, q16, pos);
     } else {
         load16_f16(static_cast<const uint16_t*>(in.k) + src, xk);
         load16_f16(static_cast<const uint16_t*>(in.v) + src, xv);
@@ -177,111 +224,118 @@ __global__ void __launch_bounds__(256) append_kernel(
 
     const size_t slab = slab_of(g, seq, pos, head);
     const uint32_t tp = pos % g.page_tokens;
-    const size_t slab_bytes = static_cast<size_t>(g.page_tokens) * D;
+    const size_t slab_elems = static_cast<size_t>(g.page_tokens) * D;
     const uint32_t d0 = q16 * 16;
-
-    // K: dims d0..d0+7 and d0+8..d0+15 are two 8-element runs of the tiled layout.
     if (g.k_f16) {
-        uint16_t* kslab = reinterpret_cast<uint16_t*>(g.k_codes) + slab * slab_bytes;
+        uint16_t* kslab = reinterpret_cast<uint16_t*>(g.k_codes) + slab * slab_elems;
         *reinterpret_cast<uint4*>(kslab + k_code_offset(tp, d0, D)) = pack8_f16(xk);
         *reinterpret_cast<uint4*>(kslab + k_code_offset(tp, d0 + 8, D)) = pack8_f16(xk + 8);
     } else {
-        int8_t* kslab = g.k_codes + slab * slab_bytes;
-        uint32_t packed[4];
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            packed[w] = (static_cast<uint32_t>(static_cast<uint8_t>(qk[4 * w]))) |
-                        (static_cast<uint32_t>(static_cast<uint8_t>(qk[4 * w + 1])) << 8) |
-                        (static_cast<uint32_t>(static_cast<uint8_t>(qk[4 * w + 2])) << 16) |
-                        (static_cast<uint32_t>(static_cast<uint8_t>(qk[4 * w + 3])) << 24);
-        }
-        *reinterpret_cast<uint2*>(kslab + k_code_offset(tp, d0, D)) = make_uint2(packed[0], packed[1]);
-        *reinterpret_cast<uint2*>(kslab + k_code_offset(tp, d0 + 8, D)) = make_uint2(packed[2], packed[3]);
+        store_k_codes16(g, slab, tp, q16, pack16_codes(qk), sk);
     }
-
-    // V: each dim is its own token-contiguous run; one element per dim.
-    if (g.v_f16) {
-        uint16_t* vslab = reinterpret_cast<uint16_t*>(g.v_codes) + slab * slab_bytes;
+    if (g.v_f16) {  // each dim is its own token-contiguous run
+        uint16_t* vslab = reinterpret_cast<uint16_t*>(g.v_codes) + slab * slab_elems;
 #pragma unroll
         for (int i = 0; i < 16; ++i) vslab[v_code_offset(tp, d0 + i, D)] = f32_to_f16_bits(xv[i]);
     } else {
-        int8_t* vslab = g.v_codes + slab * slab_bytes;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) vslab[v_code_offset(tp, d0 + i, D)] = qv[i];
-    }
-
-    if ((q16 & 1) == 0) {
-        const size_t sidx = (slab * g.page_tokens + tp) * (D / 32) + d0 / 32;
-        if (!g.k_f16) g.k_scales[sidx] = f32_to_f16_bits(sk);
-        if (!g.v_f16) g.v_scales[sidx] = f32_to_f16_bits(sv);
+        store_v_codes16(g, slab, tp, q16, pack16_codes(qv), sv);
     }
 }
 
-// Bulk append of whole 32-token groups: one workgroup per (group, kv head), one
+// Bulk append: one workgroup per (32-token group, kv head), one
 // thread per (token, 16-dim group) with the same arithmetic as append_kernel (so the
-// codes are identical), but the codes and scales are assembled in LDS and leave as
-// contiguous 16-byte stores: a 32-token group owns 32*D contiguous bytes of the K
-// slab (two 16-token tiles), 32*D of the V slab (one group) and 32*D/32 scales of
-// each kind.  base_position is a multiple of 32 and every group lies inside the
-// sequence's capacity (checked on the host).
+// codes are identical), but the codes and scales of a whole group are assembled in LDS
+// and leave as contiguous 16-byte stores: a 32-token group owns 32*D contiguous bytes of
+// the K slab (two 16-token tiles), 32*D of the V slab (one group) and 32*D/32 scales of
+// each kind.  The partial groups at either end of the rows store theirs token by token, in
+// the same launch.  Every token lies inside the sequence's capacity (checked on the host).
+// Bound: HBM, given three workgroups per CU (at two, 21.6 us below).  8195 fp32 rows with
+// the K prologue at position 77, 4 kv heads, D = 256 (85 MB): 34.2 -> 19.6 us (4.3 TB/s);
+// launches of their own for the partial groups took 13 of it.  4096 fp16 rows at position
+// 5, 8 kv heads, D = 128: 16.6 -> 8.8; whole groups alone (8192 fp16 rows at 0) 10.0 -> 10.3.
 template <bool F32>
-__global__ void __launch_bounds__(512) append_tile_kernel(Geo g, AppendIn in, uint32_t base_position,
-                                                          uint32_t seq) {
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) append_tile_kernel(Geo g, AppendIn in, uint32_t token_count,
+                                                          uint32_t base_position, uint32_t seq) {
     extern __shared__ uint4 s_tile[];
     const uint32_t D = g.head_dim;
     const uint32_t groups = D / 16;
     const uint32_t head = blockIdx.y;
     const uint32_t tl = threadIdx.x / groups;  // token within the 32-token group
     const uint32_t q16 = threadIdx.x % groups;
-    const uint32_t token = blockIdx.x * 32 + tl;
-    const uint32_t pos = base_position + token;
+    const uint32_t pos0 = (base_position / 32 + blockIdx.x) * 32;  // the group's first position
+    const uint32_t pos = pos0 + tl;
+    const bool mine = pos >= base_position && pos - base_position < token_count;
+    const uint32_t token = mine ? pos - base_position : 0;  // others compute a row and drop it
     const size_t src = (static_cast<size_t>(token) * g.kv_heads + head) * D + q16 * 16;
     float xk[16], xv[16];
     if constexpr (F32) {
-        load16_f32(static_cast<const float*>(in.k) + src, xk);
         load16_f32(static_cast<const float*>(in.v) + src, xv);
-        if (in.k_norm_weight != nullptr)
-            k_norm_rope16(xk, in.k_norm_weight, q16, groups, D, pos, in.rope_step, in.epsilon);
+        load16_f32(static_cast<const float*>(in.k) + src, xk);
     } else {
-        load16_f16(static_cast<const uint16_t*>(in.k) + src, xk);
         load16_f16(static_cast<const uint16_t*>(in.v) + src, xv);
+        load16_f16(static_cast<const uint16_t*>(in.k) + src, xk);
     }
-    int8_t qk[16], qv[16];
+    // V first: packed, its values leave their registers before K's prologue
+    uint4 vpk, kpk;
     float sk, sv;
-    quantize16(xk, qk, sk);
-    quantize16(xv, qv, sv);
+    {
+        int8_t q[16];
+        quantize16(xv, q, sv);
+        vpk = pack16_codes(q);
+    }
+    if constexpr (F32) {
+        if (in.k_norm_weight != nullptr) {
+            // The rotations of the group's 32 tokens, shared out over all threads (a rotating
+            // lane computing its own 16 keeps three quarters of the lanes idle meanwhile).
+            __shared__ float2 s_rot[32][33];  // [token][pair] (sine, cosine)
+            auto prologue = [&](auto tag) __attribute__((always_inline)) {
+                constexpr uint32_t GROUPS = decltype(tag)::value, PER = 32 / GROUPS;
+                float angle = rope_angle<31>(pos, in.rope_step, PER * q16);
+#pragma unroll
+                for (uint32_t k = 0; k < PER; ++k) {
+                    float2 sc;
+                    rope_sincos(angle, &sc.x, &sc.y);
+                    s_rot[tl][PER * q16 + k] = sc;
+                    angle *= in.rope_step;
+                }
+                // written and read by the same wave (a token's lanes): no barrier
+                const float2* rot = &s_rot[tl][16 * (q16 & 1)];
+                k_norm_rope16<GROUPS>(xk, in.k_norm_weight, q16, in.epsilon,
+                                      [&](int j) __attribute__((always_inline)) { return rot[j]; });
+            };
+            if (groups == 16) prologue(std::integral_constant<uint32_t, 16>{});
+            else prologue(std::integral_constant<uint32_t, 8>{});
+        }
+    }
+    {
+        int8_t q[16];
+        quantize16(xk, q, sk);
+        kpk = pack16_codes(q);
+    }
+    if (pos0 < base_position || pos0 + 31 - base_position >= token_count) {  // a partial group (workgroup-uniform)
+        if (mine) {
+            const size_t slab = slab_of(g, seq, pos, head);
+            store_k_codes16(g, slab, pos % g.page_tokens, q16, kpk, sk);
+            store_v_codes16(g, slab, pos % g.page_tokens, q16, vpk, sv);
+        }
+        return;
+    }
 
     uint8_t* s_k = reinterpret_cast<uint8_t*>(s_tile);  // [32*D] K codes, slab order
     uint8_t* s_v = s_k + 32 * D;                         // [32][D] V codes, token-major
     uint16_t* s_s = reinterpret_cast<uint16_t*>(s_v + 32 * D);  // [2][32][D/32] scales
     const uint32_t d0 = q16 * 16;
-    uint32_t packed[4];
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        packed[w] = (static_cast<uint32_t>(static_cast<uint8_t>(qk[4 * w]))) |
-                    (static_cast<uint32_t>(static_cast<uint8_t>(qk[4 * w + 1])) << 8) |
-                    (static_cast<uint32_t>(static_cast<uint8_t>(qk[4 * w + 2])) << 16) |
-                    (static_cast<uint32_t>(static_cast<uint8_t>(qk[4 * w + 3])) << 24);
-    }
-    *reinterpret_cast<uint2*>(s_k + k_code_offset(tl, d0, D)) = make_uint2(packed[0], packed[1]);
-    *reinterpret_cast<uint2*>(s_k + k_code_offset(tl, d0 + 8, D)) = make_uint2(packed[2], packed[3]);
+    *reinterpret_cast<uint2*>(s_k + k_code_offset(tl, d0, D)) = make_uint2(kpk.x, kpk.y);
+    *reinterpret_cast<uint2*>(s_k + k_code_offset(tl, d0 + 8, D)) = make_uint2(kpk.z, kpk.w);
     // V codes row-major here (one 16-byte store, no bank conflicts); the slab's
     // token-interleaved order is gathered on the way out.
-    uint32_t vpk[4];
-#pragma unroll
-    for (int w = 0; w < 4; ++w)
-        vpk[w] = (static_cast<uint32_t>(static_cast<uint8_t>(qv[4 * w]))) |
-                 (static_cast<uint32_t>(static_cast<uint8_t>(qv[4 * w + 1])) << 8) |
-                 (static_cast<uint32_t>(static_cast<uint8_t>(qv[4 * w + 2])) << 16) |
-                 (static_cast<uint32_t>(static_cast<uint8_t>(qv[4 * w + 3])) << 24);
-    *reinterpret_cast<uint4*>(s_v + tl * D + d0) = make_uint4(vpk[0], vpk[1], vpk[2], vpk[3]);
+    *reinterpret_cast<uint4*>(s_v + tl * D + d0) = vpk;
     if ((q16 & 1) == 0) {
         s_s[tl * (D / 32) + d0 / 32] = f32_to_f16_bits(sk);
         s_s[32 * (D / 32) + tl * (D / 32) + d0 / 32] = f32_to_f16_bits(sv);
     }
     __syncthreads();
 
-    const uint32_t pos0 = base_position + blockIdx.x * 32;
     const size_t slab = slab_of(g, seq, pos0, head);
     const uint32_t tp0 = pos0 % g.page_tokens;
     const size_t slab_bytes = static_cast<size_t>(g.page_tokens) * D;
@@ -605,18 +659,8 @@ extern "C" miikv_status miikv_plane_bytes(const miikv_view* view, uint64_t* code
     return MIIKV_OK;
 }
 
-// Token count from which a host-positioned append sends its whole 32-token groups to
-// append_tile_kernel (the partial groups at either end go through append_kernel).
+// Token count from which a host-positioned append goes to append_tile_kernel.
 constexpr uint32_t kTileAppendMin = 64;
-
-template <bool F32>
-static AppendIn advance_rows(AppendIn in, uint64_t tokens, uint32_t kv_heads, uint32_t D) {
-    const uint64_t elems = tokens * kv_heads * D;
-    const size_t esize = F32 ? sizeof(float) : sizeof(uint16_t);
-    in.k = static_cast<const char*>(in.k) + elems * esize;
-    in.v = static_cast<const char*>(in.v) + elems * esize;
-    return in;
-}
 
 template <bool F32>
 static miikv_status launch_rows(const miikv_view* view, const AppendIn& in, uint32_t rows_tokens, uint32_t base,
@@ -636,27 +680,17 @@ template <bool F32>
 static miikv_status launch_append(const miikv_view* view, const AppendIn& in, uint32_t rows_tokens, uint32_t base,
                                   uint32_t seq, const miikv_prefill_state* ps, const miikv_decode_state* ds,
                                   const uint32_t* positions, void* stream) {
-    // Positions known on the host: [head partial group][whole groups][tail partial group].
     // (The grouped store assembles q8 codes and scales; caches with an fp16 plane take
-    // the per-row kernel.)
+    // the per-row kernel, and so do positions on the device.)
     if (ps == nullptr && ds == nullptr && positions == nullptr && rows_tokens >= kTileAppendMin &&
         view->quant_mode == MIIKV_KV_Q8_Q8) {
         const uint32_t D = view->head_dim;
-        const uint32_t head = (32 - base % 32) % 32;
-        const uint32_t whole = (rows_tokens - head) / 32;
-        const uint32_t tail = rows_tokens - head - whole * 32;
-        int st = launch_rows<F32>(view, in, head, base, seq, nullptr, nullptr, nullptr, stream);
-        if (st != MIIKV_OK) return st;
-        if (whole > 0) {
-            const size_t lds = 2 * 32 * D + 2 * 32 * (D / 32) * sizeof(uint16_t);
-            hipLaunchKernelGGL(append_tile_kernel<F32>, dim3(whole, view->kv_heads), dim3(32 * (D / 16)), lds,
-                               static_cast<hipStream_t>(stream), make_geo(*view),
-                               advance_rows<F32>(in, head, view->kv_heads, D), base + head, seq);
-            st = launch_status();
-            if (st != MIIKV_OK) return st;
-        }
-        return launch_rows<F32>(view, advance_rows<F32>(in, head + 32ull * whole, view->kv_heads, D), tail,
-                                base + head + whole * 32, seq, nullptr, nullptr, nullptr, stream);
+        const uint64_t groups = (static_cast<uint64_t>(base) + rows_tokens + 31) / 32 - base / 32;
+        const size_t lds = 2 * 32 * D + 2 * 32 * (D / 32) * sizeof(uint16_t);
+        hipLaunchKernelGGL(append_tile_kernel<F32>, dim3(static_cast<uint32_t>(groups), view->kv_heads),
+                           dim3(32 * (D / 16)), lds, static_cast<hipStream_t>(stream), make_geo(*view), in,
+                           rows_tokens, base, seq);
+        return launch_status();
     }
     return launch_rows<F32>(view, in, rows_tokens, base, seq, ps, ds, positions, stream);
 }

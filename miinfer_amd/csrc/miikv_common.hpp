@@ -168,6 +168,18 @@ __device__ __forceinline__ void quantize16(const float (&x)[16], int8_t (&q)[16]
     scale_out = scale;
 }
 
+// Sixteen signed codes as packed bytes.
+__device__ __forceinline__ uint4 pack16_codes(const int8_t (&q)[16]) {
+    uint32_t w[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+        w[u] = static_cast<uint32_t>(static_cast<uint8_t>(q[4 * u])) |
+               (static_cast<uint32_t>(static_cast<uint8_t>(q[4 * u + 1])) << 8) |
+               (static_cast<uint32_t>(static_cast<uint8_t>(q[4 * u + 2])) << 16) |
+               (static_cast<uint32_t>(static_cast<uint8_t>(q[4 * u + 3])) << 24);
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
 __device__ __forceinline__ uint16_t f32_to_f16_bits(float x) {
     __half h = __float2half_rn(x);
     return __half_as_ushort(h);

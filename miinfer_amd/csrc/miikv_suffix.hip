@@ -57,18 +57,6 @@ __device__ __forceinline__ uint32_t context_keys(uint32_t host_count, const miik
     return ps ? min(host_count, ps->base_position + ps->token_count) : host_count;
 }
 
-// Sixteen signed codes as packed bytes.
-__device__ __forceinline__ uint4 pack16_codes(const int8_t (&q)[16]) {
-    uint32_t w[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-        w[u] = static_cast<uint32_t>(static_cast<uint8_t>(q[4 * u])) |
-               (static_cast<uint32_t>(static_cast<uint8_t>(q[4 * u + 1])) << 8) |
-               (static_cast<uint32_t>(static_cast<uint8_t>(q[4 * u + 2])) << 16) |
-               (static_cast<uint32_t>(static_cast<uint8_t>(q[4 * u + 3])) << 24);
-    return make_uint4(w[0], w[1], w[2], w[3]);
-}
-
 // One 32-key step of kv head blockIdx.y: 256 threads; keys at or past the context
 // end become 0 (their codes may never have been written).
 // Bound: the latency of one chain (block table, codes and scales, tiles) in short

@@ -257,3 +257,23 @@ def test_export_dequant_matches_oracle(gpu, paged):
     torch.cuda.synchronize()
     assert np.array_equal(kd.cpu().numpy(), oracle.dequantize_rows(kc, ks)[:, 100:400])
     assert np.array_equal(vd.cpu().numpy(), oracle.dequantize_rows(vc, vs)[:, 100:400])
+
+
+@pytest.mark.parametrize("base,t", [(31, 64), (33, 65), (1, 95), (0, 97), (63, 66), (32, 64)])
+def test_append_bulk_ends_inside_groups(gpu, base, t):
+    """A bulk append that starts or ends inside a 32-token group leaves the group's other
+    tokens as they were."""
+    import miinfer_amd as m
+    hk, d, n = 2, 128, 192
+    rng = np.random.default_rng(base + t)
+    cache = m.KvCache.contiguous(hk, d, n)
+    rows = [randn_f16(rng, (n, hk, d)) for _ in range(2)]
+    cache.append(*(_dev(x, gpu) for x in rows))
+    new = [randn_f16(rng, (t, hk, d)) for _ in range(2)]
+    cache.append(*(_dev(x, gpu) for x in new), base_position=base)
+    for x, y in zip(rows, new):
+        x[base:base + t] = y
+    got = _export_np(cache, 0, 0, n)
+    for i, x in enumerate(rows):
+        codes, scales = oracle.quantize_rows(x.transpose(1, 0, 2))
+        assert np.array_equal(got[2 * i], codes) and np.array_equal(got[2 * i + 1], scales)
