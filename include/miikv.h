@@ -399,6 +399,12 @@ miikv_status miikv_import_canonical(const miikv_view* view, uint32_t seq, uint32
 miikv_status miikv_copy_pages(const miikv_view* view, const int32_t* d_src_pages,
                               const int32_t* d_dst_pages, uint32_t n, void* stream);
 
+/* miikv_copy_pages with the lists in host memory, read before the call returns and passed
+ * to the device in the kernel's arguments (no upload, no allocation; may be captured).
+ * MIIKV_EINVAL, and nothing copied, for an index outside [0, num_pages). */
+miikv_status miikv_copy_pages_host(const miikv_view* view, const int32_t* src_pages, const int32_t* dst_pages,
+                                   uint32_t n, void* stream);
+
 /* Execute n device-to-device copies described by a DEVICE array of segments in
  * one launch.  Replaces the 2*48 hipMemcpyAsync calls of
  * GdnCheckpointStorage::capture/restore (src/prefill_v2/reusable_context.cpp:65-128). */

@@ -98,6 +98,7 @@ SIGNATURES = {
     "miikv_registry_set_layout_version": (ctypes.c_int, [_P, _U32, _U32]),
     "miikv_export_dequant": (ctypes.c_int, [_VP, _U32, _U32, _U32, _P, _P, _P]),
     "miikv_copy_pages": (ctypes.c_int, [_VP, _P, _P, _U32, _P]),
+    "miikv_copy_pages_host": (ctypes.c_int, [_VP, _P, _P, _U32, _P]),
     "miikv_copy_segments": (ctypes.c_int, [_P, _U32, _P]),
     "miikv_decode_state_advance": (ctypes.c_int, [_P, _P, _U32, _P, _U32, _P]),
     "miikv_clone_state": (ctypes.c_int, [_P, _P, _U64, _U32, _P]),

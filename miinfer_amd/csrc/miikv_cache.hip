@@ -1,6 +1,7 @@
 // q8_0 append, canonical export/import, page copy, segment copy and state clone.
 #include "miikv_common.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <type_traits>
@@ -557,12 +558,8 @@ __device__ __forceinline__ void copy16(uint4* __restrict__ dst, const uint4* __r
     for (uint64_t i = start; i < n16; i += stride) dst[i] = src[i];
 }
 
-// grid (blocks, n_pages): block y copies page src_pages[y] -> dst_pages[y], all four planes.
-__global__ void __launch_bounds__(256) copy_pages_kernel(Geo g, const int32_t* __restrict__ srcp,
-                                                         const int32_t* __restrict__ dstp) {
-    const uint32_t i = blockIdx.y;
-    const size_t s = static_cast<size_t>(srcp[i]);
-    const size_t d = static_cast<size_t>(dstp[i]);
+// Page s to page d, all four planes, by the gridDim.x workgroups of one blockIdx.y.
+__device__ __forceinline__ void copy_page(const Geo& g, size_t s, size_t d) {
     const uint64_t code_bytes = static_cast<uint64_t>(g.kv_heads) * g.page_tokens * g.head_dim;
     const uint64_t kbytes = code_bytes * (g.k_f16 ? 2 : 1), vbytes = code_bytes * (g.v_f16 ? 2 : 1);
     const uint64_t scale_bytes = static_cast<uint64_t>(g.kv_heads) * g.page_tokens * (g.head_dim / 32) * 2;
@@ -580,6 +577,23 @@ __global__ void __launch_bounds__(256) copy_pages_kernel(Geo g, const int32_t* _
         copy16(reinterpret_cast<uint4*>(reinterpret_cast<uint8_t*>(g.v_scales) + d * scale_bytes),
                reinterpret_cast<const uint4*>(reinterpret_cast<const uint8_t*>(g.v_scales) + s * scale_bytes),
                scale_bytes / 16, start, stride);
+}
+
+// grid (blocks, n_pages): block y copies page src_pages[y] -> dst_pages[y].
+__global__ void __launch_bounds__(256) copy_pages_kernel(Geo g, const int32_t* __restrict__ srcp,
+                                                         const int32_t* __restrict__ dstp) {
+    copy_page(g, static_cast<size_t>(srcp[blockIdx.y]), static_cast<size_t>(dstp[blockIdx.y]));
+}
+
+// The same with the list in the kernel's arguments: a fork's pairs are made on the host, and
+// an upload for each cache cost more than the copy (24 pages of 4 kv heads, D = 256: 7 us).
+constexpr uint32_t kPageList = 256;
+struct PageList {
+    int32_t src[kPageList];
+    int32_t dst[kPageList];
+};
+__global__ void __launch_bounds__(256) copy_page_list_kernel(Geo g, PageList list) {
+    copy_page(g, static_cast<size_t>(list.src[blockIdx.y]), static_cast<size_t>(list.dst[blockIdx.y]));
 }
 
 // grid (blocks, n): block y copies segment y.  16-byte path when both ends and
@@ -797,18 +811,44 @@ extern "C" miikv_status miikv_export_dequant(const miikv_view* view, uint32_t se
     return launch_status();
 }
 
+// Workgroups per copied page.
+static uint32_t page_blocks(const miikv_view* view) {
+    const uint64_t code16 = static_cast<uint64_t>(view->kv_heads) * view->page_tokens * view->head_dim / 16;
+    return static_cast<uint32_t>(std::min<uint64_t>((code16 + 255) / 256, 64));
+}
+
 extern "C" miikv_status miikv_copy_pages(const miikv_view* view, const int32_t* d_src_pages,
                                          const int32_t* d_dst_pages, uint32_t n, void* stream) {
     const int st = validate_view(view);
     if (st != MIIKV_OK) return st;
     if (n == 0) return MIIKV_OK;
     if (d_src_pages == nullptr || d_dst_pages == nullptr || n > 65535u) return MIIKV_EINVAL;
-    const uint64_t code16 = static_cast<uint64_t>(view->kv_heads) * view->page_tokens * view->head_dim / 16;
-    uint32_t blocks = static_cast<uint32_t>((code16 + 255) / 256);
-    if (blocks > 64) blocks = 64;
-    hipLaunchKernelGGL(copy_pages_kernel, dim3(blocks, n), dim3(256), 0, static_cast<hipStream_t>(stream),
+    hipLaunchKernelGGL(copy_pages_kernel, dim3(page_blocks(view), n), dim3(256), 0, static_cast<hipStream_t>(stream),
                        make_geo(*view), d_src_pages, d_dst_pages);
     return launch_status();
+}
+
+extern "C" miikv_status miikv_copy_pages_host(const miikv_view* view, const int32_t* src_pages,
+                                              const int32_t* dst_pages, uint32_t n, void* stream) {
+    const int st = validate_view(view);
+    if (st != MIIKV_OK) return st;
+    if (n == 0) return MIIKV_OK;
+    if (src_pages == nullptr || dst_pages == nullptr || n > 65535u) return MIIKV_EINVAL;
+    for (uint32_t i = 0; i < n; ++i)
+        if (src_pages[i] < 0 || dst_pages[i] < 0 || static_cast<uint32_t>(src_pages[i]) >= view->num_pages ||
+            static_cast<uint32_t>(dst_pages[i]) >= view->num_pages)
+            return MIIKV_EINVAL;
+    for (uint32_t i0 = 0; i0 < n; i0 += kPageList) {
+        PageList list{};
+        const uint32_t m = std::min(kPageList, n - i0);
+        std::copy(src_pages + i0, src_pages + i0 + m, list.src);
+        std::copy(dst_pages + i0, dst_pages + i0 + m, list.dst);
+        hipLaunchKernelGGL(copy_page_list_kernel, dim3(page_blocks(view), m), dim3(256), 0,
+                           static_cast<hipStream_t>(stream), make_geo(*view), list);
+        const int ls = launch_status();
+        if (ls != MIIKV_OK) return ls;
+    }
+    return MIIKV_OK;
 }
 
 extern "C" miikv_status miikv_copy_segments(const miikv_segment* d_segments, uint32_t n, void* stream) {

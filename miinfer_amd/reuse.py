@@ -12,7 +12,7 @@ import numpy as np
 import torch
 
 from ._lib import MIIKV_EWORKSPACE, call, check, lib
-from .kv import KvCache, _on_stream, _ptr, _stream
+from .kv import KvCache, _ptr, _stream
 
 
 class MatchResult(enum.IntEnum):
@@ -109,14 +109,14 @@ class PagePool:
 
 
 def run_page_copies(cache: KvCache, copies, stream=None) -> None:
-    """Execute [(src, dst)] physical page copies on the device in one launch."""
+    """Execute [(src, dst)] physical page copies on the device in one launch (the page
+    lists travel in its arguments)."""
     if not copies:
         return
-    dev = cache.k_codes.device
-    with _on_stream(stream):  # the page lists live until the copy has run on `stream`
-        src = torch.tensor([c[0] for c in copies], dtype=torch.int32, device=dev)
-        dst = torch.tensor([c[1] for c in copies], dtype=torch.int32, device=dev)
-    cache.copy_pages(src, dst, stream)
+    src, dst = (np.array([c[i] for c in copies], np.int32) for i in (0, 1))
+    if min(src.min(), dst.min()) < 0 or max(src.max(), dst.max()) >= cache.num_pages:
+        raise ValueError("page index out of range")
+    call("miikv_copy_pages_host", cache.view, _i32p(src), _i32p(dst), len(copies), _stream(stream))
 
 
 class RecurrentStates:

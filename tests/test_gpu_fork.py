@@ -109,3 +109,27 @@ def test_recurrent_state_clone_checkpoint_restore(gpu):
     ctx.restore(src)
     assert torch.equal(src.buf.view(torch.int32), saved.view(torch.int32))
     assert src.position == 100
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 300])
+def test_page_copies_from_host_lists(gpu, n):
+    """Page copies whose lists travel in the kernel's arguments, around the 256 pairs one
+    launch holds: every plane's pages equal their sources, the others are untouched."""
+    import miinfer_amd as m
+    from miinfer_amd import reuse
+    rng = np.random.default_rng(n)
+    pages, hk, d, pt = 640, 1, 128, 64
+    cache = m.KvCache.paged_cache(hk, d, pages, torch.zeros((1, 1), dtype=torch.int32, device=gpu), page_tokens=pt)
+    planes = (cache.k_codes, cache.v_codes, cache.k_scales, cache.v_scales)
+    for p in planes:
+        p.random_(-100, 100)
+    expect = [p.clone().view(pages, -1) for p in planes]
+    perm = rng.permutation(pages)
+    pairs = [(int(perm[i]), int(perm[n + i])) for i in range(n)]
+    reuse.run_page_copies(cache, pairs)
+    for p, e in zip(planes, expect):
+        e[[b for _, b in pairs]] = e[[a for a, _ in pairs]]
+        assert torch.equal(p.view(pages, -1), e)
+    for bad in ((0, pages), (-1, 0)):
+        with pytest.raises(ValueError):
+            reuse.run_page_copies(cache, pairs + [bad])
