@@ -1199,7 +1199,8 @@ extern "C" uint64_t miikv_suffix_workspace_bytes(const miikv_view* view, uint32_
         suffix_runs_as_decode(view, q_heads, token_count, true))
         dec = suffix_by_decode_bytes(view, q_heads, token_count, static_cast<uint32_t>(std::min<uint64_t>(cap, 0xffffffffu)));
     const SuffixPlan p = make_suffix_plan(view, q_heads, token_count, cap, true);
-    const SuffixPlan small = make_suffix_plan(view, q_heads, token_count, cap, true, 0, false, kSufWavesSmall);
+    // (the 4-wave form splits only where the 8-wave form does)
+    const SuffixPlan small = make_suffix_plan(view, q_heads, token_count, cap, p.splits > 1, 0, false, kSufWavesSmall);
     return p.tile_bytes + std::max({dec, p.part_bytes, small.part_bytes});
 }
 
