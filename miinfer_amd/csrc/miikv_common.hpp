@@ -262,6 +262,43 @@ __device__ __forceinline__ float4v mfma_16x16x16(half4 a, half4 b, float4v c) {
     return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
 }
 
+__device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// This wave's LDS reads have returned (what they read may be overwritten).
+__device__ __forceinline__ void lds_reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+// Wait until at most N vector-memory operations of this wave are outstanding.
+template <uint32_t N>
+__device__ __forceinline__ void wait_vmem_le() {
+    static_assert(N < 64, "vmcnt holds 6 bits");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
+}
+
+// 16 bytes per lane from `src` (per lane) to LDS at `lds` + 16 * lane (`lds` wave-uniform;
+// NT: nontemporal).  In asm: the compiler waits for every copy that it knows of at each
+// barrier and LDS read; here the caller counts them (wait_vmem_le).
+template <bool NT = false>
+__device__ __forceinline__ void copy_to_lds(const void* src, uint32_t lds) {
+    if constexpr (NT)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt"
+                     :
+                     : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(src)
+                     : "memory", "m0");
+    else
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                     :
+                     : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(src)
+                     : "memory", "m0");
+}
+__device__ __forceinline__ uint32_t lds_offset(const void* p) {
+    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void*)p));
+}
+
+// A word that no kernel running meanwhile writes, at a wave-uniform address, through the
+// scalar cache: its wait holds up no vector load or copy.
+template <typename T>
+__device__ __forceinline__ T scalar_load(const T* p) {
+    return *reinterpret_cast<const __attribute__((address_space(4))) T*>(reinterpret_cast<uintptr_t>(p));
+}
+
 inline int hip_status(hipError_t e) { return e == hipSuccess ? MIIKV_OK : -static_cast<int>(e); }
 
 }  // namespace miikv

@@ -140,6 +140,12 @@ __device__ __forceinline__ float wave_max_xor_16_32(float x) {
     return rows_reduce(x, MaxOp{});
 }
 
+// split_length by a scalar load (b wave-uniform).
+__device__ __forceinline__ uint32_t split_length_scalar(const SplitArgs& a, uint32_t b) {
+    const uint32_t L = (a.len_ptr ? scalar_load(a.len_ptr + static_cast<size_t>(b) * a.len_stride) : 0u) + a.len_add + b * a.len_bstep;
+    return min(L, a.max_context);
+}
+
 // A value every lane of the wave holds, in scalar registers.
 __device__ __forceinline__ unsigned long long uniform64(unsigned long long x) {
     const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(x));
@@ -311,8 +317,19 @@ constexpr uint32_t decode_waves_per_eu() {
 // per score (a constant DPP shift); the fp16-query register budget and occupancy then
 // hold.  Otherwise (G > 8) the lo parts are a second fragment set and a second MFMA per
 // block.
+// LDS (D = 256): the wave's step lives in LDS, copied there without registers, not in
+// registers: K's half is refilled for the next step as soon as the scores have read it,
+// V's half after the values, so a wave always has one of them in flight (a step's codes and
+// scales take 68 registers, too many for a second set beside O and the query at two waves
+// per SIMD), and its first step is asked for before the query and the length arrive.
+// Bound: the latency of that chain, then HBM.  24q/4kv, one sequence, us a step with the
+// append, registers -> LDS: q8 200 / 4096 / 16384 / 32768 keys 10.8 -> 10.4 / 12.2 -> 11.9 /
+// 17.4 -> 16.0 / 23.4 -> 21.3 (3.3 TB/s), 9001 of at most 16384 with the K prologue 18.4 ->
+// 16.5; fp16 planes 4096 / 16384 / 32768 16.2 -> 15.8 / 24.2 -> 23.0 / 36.1 -> 32.2 (4.2 TB/s).
+// Batches over one resident round (STREAM: 188.9 -> 199.2 at config 3) and row sets of one
+// sequence (CACHED: 25.6 -> 26.4 for 5 tokens over 8187) stay with registers.
 template <uint32_t D, bool QF32, bool APPEND, bool KF16 = false, bool VF16 = false, bool QPAIR = false,
-          bool CACHED = false, bool STREAM = false>
+          bool CACHED = false, bool STREAM = false, bool LDS = false>
 __global__ void __launch_bounds__(64 * kWavesPerWg)
 __attribute__((amdgpu_waves_per_eu(decode_waves_per_eu<D, QF32 && !QPAIR, KF16, VF16>())))
 decode_kernel(SplitArgs a) {
@@ -324,6 +341,8 @@ decode_kernel(SplitArgs a) {
     // with column sums, or exactly (perm + subtract): the fold costs NB accumulators.
     constexpr bool kLo = QF32 && !QPAIR;  // separate lo fragments and MFMAs
     static_assert(!QPAIR || QF32, "QPAIR splits an fp32 query");
+    constexpr bool kLds = LDS;
+    static_assert(!LDS || (D == 256 && !CACHED && !STREAM && KF16 == VF16), "instances of the LDS form");
     constexpr bool kVBias = DecodeTuning<D, kLo>::vbias && !VF16;
     static_assert(!APPEND || (!KF16 && !VF16), "the fused append stores q8 rows");
     extern __shared__ float smem[];
@@ -341,11 +360,17 @@ decode_kernel(SplitArgs a) {
             return;
         }
     }
-    const uint32_t wave = STREAM ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
+    const uint32_t wave = STREAM || kLds ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
     const uint32_t G = a.group;
     const Geo& geo = a.g;
 
     const size_t slab_bytes = static_cast<size_t>(geo.page_tokens) * D;
+
+    // LDS form: the wave's step, in the cache's order: K codes, V codes, K scales, V scales.
+    constexpr uint32_t kKB = kChunk * D * (KF16 ? 2 : 1), kVB = kChunk * D * (VF16 ? 2 : 1), kSB = kChunk * NB * 2;
+    constexpr uint32_t kBuf = kKB + kVB + 2 * kSB;
+    __shared__ __align__(16) uint8_t s_step[kLds ? kWavesPerWg : 1][kLds ? kBuf : 16];
+    uint8_t* const buf = s_step[kLds ? wave : 0];
 
     // Registers of one 32-token step: two K tiles, one V group, their scales.
     struct Step {
@@ -374,7 +399,7 @@ decode_kernel(SplitArgs a) {
     uint32_t ld_tok = first * kChunk;
     uint32_t ld_tp = ld_tok % geo.page_tokens;
     size_t ld_slab = 0;
-    if (n_max > 0) ld_slab = slab_of_clamped(geo, b, ld_tok, h);
+    if (!kLds && n_max > 0) ld_slab = slab_of_clamped(geo, b, ld_tok, h);
     auto load_step = [&](Step& st) {
         if (ld_tp >= geo.page_tokens) {
             ld_tp = ld_tok % geo.page_tokens;
@@ -406,8 +431,42 @@ decode_kernel(SplitArgs a) {
         ld_tp += stride * kChunk;
     };
 
+    // LDS form: the next step's K half (codes after their scales), then its V half.  Each is
+    // kKOps (kVOps) copies of 16 bytes per lane.
+    constexpr uint32_t kKOps = kKB / 1024 + (KF16 ? 0 : 1), kVOps = kVB / 1024 + (VF16 ? 0 : 1);
+    const uint32_t buf_off = lds_offset(buf);
+    auto copy_kb = [&](const void* src, uint32_t off, uint32_t chunks) __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t c = 0; c < chunks; ++c)  // nontemporal: each byte is read once
+            copy_to_lds<!CACHED>(static_cast<const char*>(src) + c * 1024 + lane * 16, buf_off + off + c * 1024);
+    };
+    auto copy_scales = [&](const uint16_t* src, uint32_t off) __attribute__((always_inline)) {
+        if (lane < kSB / 16) copy_to_lds(reinterpret_cast<const char*>(src) + lane * 16, buf_off + off);
+    };
+    auto find_slab = [&]() __attribute__((always_inline)) {  // slab_of_clamped, by a scalar load
+        uint32_t page = 0;
+        if (geo.layout == MIIKV_LAYOUT_PAGED)
+            page = min(static_cast<uint32_t>(scalar_load(geo.table + static_cast<size_t>(b) * geo.table_stride +
+                                                         ld_tok / geo.page_tokens)), geo.num_pages - 1);
+        return static_cast<size_t>(page) * geo.kv_heads + h;
+    };
+    auto copy_k = [&]() __attribute__((always_inline)) {
+        if (ld_tp >= geo.page_tokens) {
+            ld_tp = ld_tok % geo.page_tokens;
+            ld_slab = find_slab();
+        }
+        if constexpr (!KF16) copy_scales(geo.k_scales + (ld_slab * geo.page_tokens + ld_tp) * NB, kKB + kVB);
+        copy_kb(geo.k_codes + (ld_slab * slab_bytes + static_cast<size_t>(ld_tp) * D) * (KF16 ? 2 : 1), 0, kKB / 1024);
+    };
+    auto copy_v = [&]() __attribute__((always_inline)) {
+        if constexpr (!VF16) copy_scales(geo.v_scales + (ld_slab * geo.page_tokens + ld_tp) * NB, kKB + kVB + kSB);
+        copy_kb(geo.v_codes + (ld_slab * slab_bytes + static_cast<size_t>(ld_tp) * D) * (VF16 ? 2 : 1), kKB, kVB / 1024);
+        ld_tok += stride * kChunk;
+        ld_tp += stride * kChunk;
+    };
+
     // Ring of kRing step buffers; the first kRing-1 are loaded before L is known.
-    constexpr uint32_t kRing = (KF16 || VF16) ? (D == 128 && !kLo ? MIIKV_RING_F16_D128 : 1u) : DecodeTuning<D, kLo>::ring;
+    constexpr uint32_t kRing = kLds ? 1u : (KF16 || VF16) ? (D == 128 && !kLo ? MIIKV_RING_F16_D128 : 1u) : DecodeTuning<D, kLo>::ring;
     Step S[kRing];
 #pragma unroll
     for (uint32_t r = 0; r + 1 < kRing; ++r)
@@ -435,9 +494,19 @@ decode_kernel(SplitArgs a) {
             }
         }
     }
-    const uint32_t L = split_length(a, b);
+    if constexpr (kLds) {
+        if (n_max > 0) {
+            ld_slab = find_slab();
+            copy_k();
+            copy_v();
+        }
+    }
+    const uint32_t L = kLds ? split_length_scalar(a, b) : split_length(a, b);
     // includes L == 0 (the combine kernel writes zeros)
-    if (!STREAM && split >= split_count(L, a.cpw)) return;
+    if (!STREAM && split >= split_count(L, a.cpw)) {
+        if constexpr (kLds) wait_vmem();  // the LDS must not be given up under a copy
+        return;
+    }
 
     // ---- Q fragments (B operand of the QK MFMA): lane (g4, n) holds head n,
     // dims 32*blk + 8*g4 .. +7 of every block.  Codes enter the MFMA as fp16
@@ -510,16 +579,33 @@ decode_kernel(SplitArgs a) {
     const uint32_t n_steps = first < nsteps ? min(n_max, (nsteps - first + stride - 1) / stride) : 0;
     // Per-wave LDS staging of one step's scales: [K: 32*NB][V: 32*NB] fp16.  Each lane
     // loads NB/2 scales (no redundancy) and re-reads the 4*NB it needs from LDS.
-    uint16_t* s_sc = reinterpret_cast<uint16_t*>(smem + 32 * kWavesPerWg + kWavesPerWg * G * D) + wave * (2 * kChunk * NB);
+    uint16_t* s_sc = kLds ? reinterpret_cast<uint16_t*>(buf + kKB + kVB)
+                          : reinterpret_cast<uint16_t*>(smem + 32 * kWavesPerWg + kWavesPerWg * G * D) + wave * (2 * kChunk * NB);
+    auto k_frag = [&](const Step& st, uint32_t J, uint32_t cc, uint32_t e) __attribute__((always_inline)) {
+        if constexpr (kLds) {
+            constexpr uint32_t KE = KF16 ? 2 : 1;
+            return *reinterpret_cast<const uint4*>(buf + KE * (J * 16 * D + cc * 1024 + lane * 16) + 16 * e);
+        } else {
+            return st.k[J][cc][e];
+        }
+    };
+    auto v_frag = [&](const Step& st, uint32_t mt) __attribute__((always_inline)) {
+        using VT = typename std::conditional<VF16, uint4, uint2>::type;
+        if constexpr (kLds) return *reinterpret_cast<const VT*>(buf + kKB + (VF16 ? 2 : 1) * ((16 * mt + n) * 32 + g4 * 8));
+        else return reinterpret_cast<const VT&>(st.v[mt]);
+    };
 
     // A step that reaches past L (only the sequence's last) is masked under a
     // wave-uniform branch: its scores go to -inf and its V scales to 0 (the memory
     // past L may hold anything, including non-finite scales).
-    auto compute_step = [&](uint32_t c, const Step& st) __attribute__((always_inline)) {
+    // LDS form: `next` is set where a further step follows; the step's own halves have to
+    // have landed, the next step's K half may be in flight beside its V half.
+    auto compute_step = [&](uint32_t c, const Step& st, bool next) __attribute__((always_inline)) {
         const uint32_t tok0 = c * kChunk;
         const bool tail = tok0 + kChunk > Lc_lo;
-        if constexpr (!KF16) *reinterpret_cast<ScaleVec*>(s_sc + lane * (NB / 2)) = st.ks;
-        if constexpr (!VF16) {
+        if constexpr (kLds) wait_vmem_le<kVOps>();
+        if constexpr (!KF16 && !kLds) *reinterpret_cast<ScaleVec*>(s_sc + lane * (NB / 2)) = st.ks;
+        if constexpr (!VF16 && !kLds) {
             ScaleVec vsv = st.vs;
             if (tail && tok0 + lane / 2 >= Lc) vsv = ScaleVec{};
             *reinterpret_cast<ScaleVec*>(s_sc + kChunk * NB + lane * (NB / 2)) = vsv;
@@ -534,8 +620,8 @@ decode_kernel(SplitArgs a) {
                 float4v c = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (uint32_t cc = 0; cc < NC; ++cc) {
-                    const half8 a0 = __builtin_bit_cast(half8, st.k[J][cc][0]);  // block 2cc
-                    const half8 a1 = __builtin_bit_cast(half8, st.k[J][cc][KF16 ? 1 : 0]);  // block 2cc+1
+                    const half8 a0 = __builtin_bit_cast(half8, k_frag(st, J, cc, 0));  // block 2cc
+                    const half8 a1 = __builtin_bit_cast(half8, k_frag(st, J, cc, KF16 ? 1 : 0));  // block 2cc+1
                     c = mfma_16x16x32(a0, qf[2 * cc], c);
                     c = mfma_16x16x32(a1, qf[2 * cc + 1], c);
                     if (kLo) {
@@ -561,7 +647,7 @@ decode_kernel(SplitArgs a) {
             float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (uint32_t cc = 0; cc < NC; ++cc) {
-                const uint4 w = st.k[J][cc][0];
+                const uint4 w = k_frag(st, J, cc, 0);
                 const half8 a0 = codes8_to_half8_biased(w.x, w.y);  // block 2cc
                 const half8 a1 = codes8_to_half8_biased(w.z, w.w);  // block 2cc+1
                 const float b0 = -kbias[2 * cc], b1 = -kbias[2 * cc + 1];
@@ -584,6 +670,13 @@ decode_kernel(SplitArgs a) {
 #pragma unroll
             for (uint32_t i = 0; i < 4; ++i) {
                 s[J][i] = acc[i] * a.scale_log2;
+            }
+        }
+
+        if constexpr (kLds) {
+            if (next) {  // K's half has been read: refill it
+                lds_reads_done();
+                copy_k();
             }
         }
 
@@ -629,6 +722,13 @@ decode_kernel(SplitArgs a) {
             }
         l_run += psum;
 
+        if constexpr (kLds) {
+            if (next) wait_vmem_le<kKOps>();
+            else wait_vmem();
+            if constexpr (!VF16)
+                if (tail && tok0 + lane / 2 >= Lc) *reinterpret_cast<ScaleVec*>(s_sc + kChunk * NB + lane * (NB / 2)) = ScaleVec{};
+        }
+
         // ---- O^T += V^T * (P^T scaled per block); V codes enter as (code + 1152), the
         // bias is removed at the end with the column sums accumulated in vbias.
         if constexpr (VF16) {
@@ -641,7 +741,7 @@ decode_kernel(SplitArgs a) {
                 for (uint32_t i = 0; i < 4; ++i) pb[i] = static_cast<_Float16>(s[J][i]);
 #pragma unroll
                 for (uint32_t mt = 0; mt < NM; ++mt) {
-                    const uint4 w = reinterpret_cast<const uint4&>(st.v[mt]);
+                    const uint4 w = v_frag(st, mt);
                     half4 va = __builtin_bit_cast(half4, J == 0 ? make_uint2(w.x, w.y) : make_uint2(w.z, w.w));
                     if (tail) {
 #pragma unroll
@@ -669,7 +769,7 @@ decode_kernel(SplitArgs a) {
 #pragma unroll
                 for (uint32_t sub = 0; sub < 2; ++sub) {
                     const uint32_t mt = 2 * blk + sub;
-                    const uint2 vw = reinterpret_cast<const uint2&>(st.v[mt]);
+                    const uint2 vw = v_frag(st, mt);
                     const uint32_t word = J == 0 ? vw.x : vw.y;
                     if constexpr (kVBias) O[mt] = mfma_16x16x16(codes4_to_half4_biased(word), pb, O[mt]);
                     else O[mt] = mfma_16x16x16(codes4_to_half4(word), pb, O[mt]);
@@ -679,6 +779,17 @@ decode_kernel(SplitArgs a) {
         }
     };
 
+    if constexpr (kLds) {
+        for (uint32_t i = 0; i < n_steps; ++i) {
+            const bool next = i + 1 < n_steps;
+            compute_step(first + i * stride, S[0], next);
+            if (next) {
+                lds_reads_done();
+                copy_v();
+            }
+        }
+        wait_vmem();  // a first step that turned out to hold no key
+    } else
     // Software pipeline over the local steps [0, n_steps): while step i computes, the
     // loads of steps i+1 .. i+kRing-1 are in flight (fully unrolled so S[] stays in
     // registers).
@@ -687,7 +798,7 @@ decode_kernel(SplitArgs a) {
         for (uint32_t r = 0; r < kRing; ++r) {
             if (i + r >= n_steps) break;
             if (i + r + kRing - 1 < n_steps) load_step(S[(r + kRing - 1) % kRing]);
-            compute_step(first + (i + r) * stride, S[r]);
+            compute_step(first + (i + r) * stride, S[r], false);
         }
     }
     if constexpr (kVBias) {
@@ -702,7 +813,12 @@ decode_kernel(SplitArgs a) {
     l_run = rows_reduce(l_run, AddOp{});
     float* s_m = smem;                          // [waves][16]
     float* s_l = smem + 16 * kWavesPerWg;       // [waves][16]
-    float4* s_O = reinterpret_cast<float4*>(smem + 32 * kWavesPerWg);  // [waves][NM][4 g4][G]
+    // [waves][NM][4 g4][G]; LDS form: each wave's in its own step buffer
+    auto o_slot = [&](uint32_t w, uint32_t i) __attribute__((always_inline)) {
+        if constexpr (kLds) return reinterpret_cast<float4*>(s_step[w]) + i;
+        else return reinterpret_cast<float4*>(smem + 32 * kWavesPerWg) + w * (NM * 4 * G) + i;
+    };
+    static_assert(!kLds || 16 * D * 4 <= kBuf, "O of 16 columns fits the step buffer");
     if (g4 == 0) {
         s_m[wave * 16 + n] = m_run;
         s_l[wave * 16 + n] = l_run;
@@ -710,7 +826,7 @@ decode_kernel(SplitArgs a) {
     if (n < G) {
 #pragma unroll
         for (uint32_t mt = 0; mt < NM; ++mt)
-            s_O[((wave * NM + mt) * 4 + g4) * G + n] = make_float4(O[mt][0], O[mt][1], O[mt][2], O[mt][3]);
+            *o_slot(wave, (mt * 4 + g4) * G + n) = make_float4(O[mt][0], O[mt][1], O[mt][2], O[mt][3]);
     }
     __syncthreads();
 
@@ -732,7 +848,7 @@ decode_kernel(SplitArgs a) {
         for (uint32_t w = 0; w < kWavesPerWg; ++w) {
             if (mw[w] == -INFINITY) continue;
             const float f = exp2_safe(mw[w] - M);
-            const float4 v = s_O[((w * NM + mt) * 4 + gq) * G + hn];
+            const float4 v = *o_slot(w, (mt * 4 + gq) * G + hn);
             o.x += v.x * f;
             o.y += v.y * f;
             o.z += v.z * f;
@@ -964,6 +1080,13 @@ constexpr uint32_t kRowsetColsF32 = MIIKV_ROWSET_COLS_F32;
 #define MIIKV_DECODE_QPAIR 1
 #endif
 namespace {
+// decode_kernel's LDS form (q8 planes, or fp16 planes from 4096 keys on: 200 / 1000 keys run
+// 13.9 / 14.6 us from registers, 14.5 / 14.9 from LDS), for launches that are neither
+// streamed nor row sets of one sequence.
+bool steps_in_lds(const SplitArgs& a, uint32_t D) {
+    if (D != 256 || a.stream_wgs != 0 || a.rowset_order) return false;
+    return !a.g.k_f16 || a.max_context >= 4096;
+}
 template <uint32_t D, bool F32, bool APP, bool KF, bool VF>
 void launch_decode_t(dim3 grid, size_t lds, hipStream_t s, const SplitArgs& a) {
     // An fp32 query of up to 8 heads per kv head pairs its lo parts into the spare columns
@@ -989,6 +1112,18 @@ void launch_decode_t(dim3 grid, size_t lds, hipStream_t s, const SplitArgs& a) {
             hipLaunchKernelGGL((decode_kernel<D, F32, APP, KF, VF, false, false, true>), grid, dim3(64 * kWavesPerWg),
                                lds, s, a);
         return;
+    }
+    if constexpr (D == 256 && KF == VF) {
+        if (steps_in_lds(a, D)) {
+            const size_t ml = 32 * kWavesPerWg * sizeof(float);  // all but (m, l) is in the step buffers
+            if (pair)
+                hipLaunchKernelGGL((decode_kernel<D, F32, APP, KF, VF, F32, false, false, true>), grid,
+                                   dim3(64 * kWavesPerWg), ml, s, a);
+            else
+                hipLaunchKernelGGL((decode_kernel<D, F32, APP, KF, VF, false, false, false, true>), grid,
+                                   dim3(64 * kWavesPerWg), ml, s, a);
+            return;
+        }
     }
     if (pair)
         hipLaunchKernelGGL((decode_kernel<D, F32, APP, KF, VF, F32>), grid, dim3(64 * kWavesPerWg), lds, s, a);
@@ -1128,8 +1263,7 @@ static miikv_status decode_impl(const miikv_view* view, const NewRows& rows,
     a.epsilon = rows.epsilon;
     a.q_f32 = q_dtype == MIIKV_DTYPE_F32;
 
-    const size_t lds = decode_lds_bytes(G, view->head_dim);
-    if (lds > 64 * 1024) return MIIKV_EUNSUPPORTED;
+    if (decode_lds_bytes(G, view->head_dim) > 64 * 1024) return MIIKV_EUNSUPPORTED;
     // One workgroup per possible (sequence, kv head, split) work item, plus one per
     // (sequence, kv head) for the new token of the fused append.
     // (A streamed plan: its workgroups instead of the splits.)
@@ -1140,6 +1274,7 @@ static miikv_status decode_impl(const miikv_view* view, const NewRows& rows,
                    (rows.any() ? static_cast<uint64_t>(view->kv_heads) * batch : 0);
     if (rs != nullptr) wgs = (wgs + 7) / 8 * 8;  // XCD-ordered items: a whole number of rounds over the XCDs
     if (wgs > 0x7fffffffu) return MIIKV_EINVAL;
+    const size_t lds = decode_lds_bytes(G, view->head_dim);
     a.batch = batch;
     const dim3 grid(static_cast<uint32_t>(wgs));
     hipStream_t s = static_cast<hipStream_t>(stream);

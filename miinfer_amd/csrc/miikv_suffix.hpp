@@ -118,26 +118,6 @@ __device__ __forceinline__ float sfx_exp2(float x) { return __builtin_amdgcn_exp
 __device__ __forceinline__ float16v mfma_32x32x16(half8 a, half8 b, float16v c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
-__device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-// Wait until at most N vector-memory operations of this wave are outstanding.
-template <uint32_t N>
-__device__ __forceinline__ void wait_vmem_le() {
-    static_assert(N < 64, "vmcnt holds 6 bits");
-    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
-}
-
-// 16 bytes per lane from `src` (per lane) to LDS at `lds` + 16 * lane (`lds` wave-uniform).
-// In asm: the compiler drains every load that it knows of at a barrier, these copies too;
-// here the caller counts them (wait_vmem_le).
-__device__ __forceinline__ void copy_to_lds(const void* src, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                 :
-                 : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(src)
-                 : "memory", "m0");
-}
-__device__ __forceinline__ uint32_t lds_offset(const void* p) {
-    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void*)p));
-}
 // Workgroup barrier after this wave's LDS reads have returned; copies stay in flight.
 __device__ __forceinline__ void lds_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");

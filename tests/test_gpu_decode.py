@@ -488,3 +488,34 @@ def test_decode_streamed_batch_edges(gpu, hq, hk, d, f32, fused):
             continue
         expect = oracle.attention_q8(q[s].astype(np.float32), *refs[s], n, hq, 1 / math.sqrt(d))
         assert_attention_close(out[s], expect, f"seq {s} L={n}")
+
+
+@pytest.mark.parametrize("mode", ["q8", "f16"])
+@pytest.mark.parametrize("hq,paged,length,cap", [(24, False, 4097, 16384), (24, True, 12300, 12544), (48, True, 8191, 8192),
+                                                 (4, False, 33, 16384), (24, False, 16384, 16384)])
+def test_decode_d256_steps_in_lds(gpu, mode, hq, paged, length, cap):
+    """head_dim 256, one sequence: steps held in LDS over several steps per wave, waves whose
+    first step lies past the context, page changes, more than 8 heads per kv head with an
+    fp32 query (its lo parts as a second fragment set), against float64 attention over the
+    dequantised cache."""
+    import miinfer_amd as m
+    from miinfer_amd import _lib
+    hk, d = 4, 256
+    rng = np.random.default_rng(length)
+    quant = _lib.KV_Q8_Q8 if mode == "q8" else _lib.KV_FP16_FP16
+    if paged:
+        table = _dev(rng.permutation(cap // 256).astype(np.int32)[None, :], gpu)
+        cache = m.KvCache.paged_cache(hk, d, cap // 256, table, quant_mode=quant)
+    else:
+        cache = m.KvCache.contiguous(hk, d, cap, quant_mode=quant)
+        for t in (cache.k_codes, cache.v_codes) if mode == "f16" else (cache.k_scales, cache.v_scales):
+            t.view(torch.float16).fill_(float("nan"))  # past the context anything may stand
+    cache.append(_dev(randn_f16(rng, (length, hk, d)), gpu), _dev(randn_f16(rng, (length, hk, d)), gpu))
+    k, v = (x.double() for x in cache.export_dequant(0, 0, length))
+    for dtype in (torch.float16, torch.float32):
+        q = _dev(rng.standard_normal((1, hq, d)).astype(np.float32), gpu).to(dtype)
+        out, _ = m.decode_attention(cache, q, lengths=_dev(np.array([length], np.int32), gpu), max_context=cap)
+        for h in range(hq):
+            s = k[h // (hq // hk)] @ q[0, h].double() / math.sqrt(d)
+            expect = torch.softmax(s, 0) @ v[h // (hq // hk)]
+            assert_attention_close(out[0, h].cpu().numpy(), expect.cpu().numpy(), f"{dtype} head {h}")
