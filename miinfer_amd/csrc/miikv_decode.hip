@@ -481,7 +481,8 @@ decode_kernel(SplitArgs a) {
         // packed tokens (a short suffix): column qh is token pack*b + qh / Gt, head qh % Gt
         const uint32_t Gt = a.pack == 1 ? G : G / a.pack;
         const uint32_t tp = a.pack == 1 ? 0u : qh / Gt;
-        const size_t qrow = ((static_cast<size_t>(b) * a.pack + tp) * a.q_heads + static_cast<size_t>(h) * Gt +
+        const uint32_t tq = a.pack == 1 || packed_context(a, b, tp) > a.max_context ? 0u : tp;  // past the suffix: any
+        const size_t qrow = ((static_cast<size_t>(b) * a.pack + tq) * a.q_heads + static_cast<size_t>(h) * Gt +
                              (qh - tp * Gt)) * D;
 #pragma unroll
         for (uint32_t blk = 0; blk < NB; ++blk) {
@@ -572,10 +573,12 @@ decode_kernel(SplitArgs a) {
     // by append_record: masked) has its own record.
     const uint32_t Lc = APPEND ? L - 1 : L;
     const uint32_t nsteps = (Lc + kChunk - 1) / kChunk;
-    // Packed tokens: column n's context is shorter by the packed tokens after its own
-    // (Lc_col); steps past Lc_lo, the shortest, mask per column.
-    const uint32_t Lc_lo = Lc - (a.pack - 1);
-    const uint32_t Lc_col = a.pack == 1 ? Lc : Lc - (a.pack - 1 - min(n, G - 1) / (G / a.pack));
+    // Packed tokens: column n's context is shorter by the packed tokens after its own (the
+    // last row set's, some of them past the suffix, counted from its full length); steps
+    // past Lc_lo, the shortest, mask per column.
+    const uint32_t Lc_full = a.pack == 1 ? Lc : a.len_add + b * a.len_bstep;
+    const uint32_t Lc_lo = Lc_full - (a.pack - 1);
+    const uint32_t Lc_col = a.pack == 1 ? Lc : min(Lc, packed_context(a, b, min(n, G - 1) / (G / a.pack)));
     const uint32_t n_steps = first < nsteps ? min(n_max, (nsteps - first + stride - 1) / stride) : 0;
     // Per-wave LDS staging of one step's scales: [K: 32*NB][V: 32*NB] fp16.  Each lane
     // loads NB/2 scales (no redundancy) and re-reads the 4*NB it needs from LDS.
@@ -1180,7 +1183,7 @@ struct RowSets {
     uint32_t len_add;
     const uint32_t* count_ptr;
     uint32_t seq;
-    uint32_t pack;  // tokens per row set (divides batch; no count_ptr when > 1)
+    uint32_t pack;  // tokens per row set (no len_ptr or count_ptr when > 1)
 };
 
 static miikv_status decode_impl(const miikv_view* view, const NewRows& rows,
@@ -1193,10 +1196,10 @@ static miikv_status decode_impl(const miikv_view* view, const NewRows& rows,
     if (st != MIIKV_OK) return st;
     if (q == nullptr || batch == 0 || q_heads == 0 || q_heads % view->kv_heads != 0 || !std::isfinite(scale))
         return MIIKV_EINVAL;
-    // packed tokens: batch / pack row sets of pack * G columns
+    // packed tokens: row sets of pack * G columns, the last one's maybe not all used
     const uint32_t pack = rs != nullptr ? rs->pack : 1u;
-    if (pack == 0 || batch % pack != 0 || (pack > 1 && rs->count_ptr != nullptr)) return MIIKV_EINVAL;
-    batch /= pack;
+    if (pack == 0 || (pack > 1 && (rs->count_ptr != nullptr || rs->len_ptr != nullptr))) return MIIKV_EINVAL;
+    batch = (batch + pack - 1) / pack;
     const uint32_t G = q_heads / view->kv_heads * pack;
     if (G > 16) return MIIKV_EUNSUPPORTED;
     if (q_dtype != MIIKV_DTYPE_F16 && q_dtype != MIIKV_DTYPE_F32) return MIIKV_EINVAL;
@@ -1310,19 +1313,29 @@ namespace miikv {
 // is row set t with context P + t + 1 (the cache already holds the suffix's rows).
 // Each row set streams its context once, so this pays for few tokens only; it
 // serves miikv_suffix_attn below a token-count threshold (miikv_suffix.hip).
-// Tokens per row set: the largest divisor of token_count whose columns (tokens x
-// query heads per kv head) fit the 16 of the MFMA and the kernel's LDS; with a device
-// token count, 1.
+// Tokens per row set: as many as have columns (tokens x query heads per kv head) in the 16
+// of the MFMA and fit the kernel's LDS; with a device token count, 1.
 bool decode_columns_fit(uint32_t G, uint32_t D) { return G <= 16 && decode_lds_bytes(G, D) <= 64 * 1024; }
 
 // max_cols: 16 (the MFMA's columns), or 8 for an fp32 query, whose lo parts then ride
 // in the other 8 columns (one MFMA per block at the fp16-query register budget).
+// ragged: the last row set may be less full than the others: as few row sets as the
+// columns allow, of about equal size (7 tokens of 4 heads per kv head: 2 row sets instead
+// of 7).  Over 8000 keys, us with the store: 32q/8kv/D128 5 / 7 / 11 tokens 27.1 -> 20.0 /
+// 26.1 -> 21.2 / 39.7 -> 23.2; 24q/4kv/D256 5 / 7 / 11 26.1 -> 25.6 / 29.3 -> 26.1 / 34.6 -> 30.7.
+// (Whether a suffix runs as decodes at all is still decided by the even packing.)
 uint32_t suffix_pack(const miikv_view* view, uint32_t q_heads, uint32_t token_count, bool device_count,
-                     uint32_t max_cols) {
+                     uint32_t max_cols, bool ragged) {
     const uint32_t G = q_heads / view->kv_heads;
     if (device_count || G == 0 || G > 16) return 1;
-    for (uint32_t p = std::min<uint32_t>(max_cols / G, token_count); p > 1; --p)
-        if (token_count % p == 0 && decode_lds_bytes(p * G, view->head_dim) <= 64 * 1024) return p;
+    for (uint32_t p = std::min<uint32_t>(max_cols / G, token_count); p > 1; --p) {
+        if (decode_lds_bytes(p * G, view->head_dim) > 64 * 1024) continue;
+        if (token_count % p == 0) return p;
+        if (ragged) {
+            const uint32_t sets = (token_count + p - 1) / p;
+            return (token_count + sets - 1) / sets;
+        }
+    }
     return 1;
 }
 
@@ -1330,9 +1343,9 @@ uint64_t suffix_by_decode_bytes(const miikv_view* view, uint32_t q_heads, uint32
     // the largest of the packed plans (fp16 and fp32 queries, host token count) and the
     // unpacked one (device count)
     uint64_t most = 0;
-    for (const uint32_t pk : {1u, suffix_pack(view, q_heads, token_count, false, 16),
-                              suffix_pack(view, q_heads, token_count, false, kRowsetColsF32)}) {
-        const Plan p = make_plan(view, q_heads * pk, token_count / pk, bound, kRowsetMaxCpw, true);
+    for (const uint32_t pk : {1u, suffix_pack(view, q_heads, token_count, false, 16, true),
+                              suffix_pack(view, q_heads, token_count, false, kRowsetColsF32, true)}) {
+        const Plan p = make_plan(view, q_heads * pk, (token_count + pk - 1) / pk, bound, kRowsetMaxCpw, true);
         most = std::max(most, p.counter_bytes + p.part_bytes);
     }
     return most;
@@ -1353,7 +1366,7 @@ miikv_status suffix_by_decode(const miikv_view* view, const void* q, uint32_t q_
     // fragment set (T = 2: 16.6 against 17.2 us; the exact route at T = 512: 790
     // against 963 us, where twice the row sets' operand conversions cost more).
     const bool pair_cols = q_dtype == MIIKV_DTYPE_F32 && token_count >= 4 && token_count <= 16;
-    rs.pack = suffix_pack(view, q_heads, token_count, prefill_state != nullptr, pair_cols ? kRowsetColsF32 : 16u);
+    rs.pack = suffix_pack(view, q_heads, token_count, prefill_state != nullptr, pair_cols ? kRowsetColsF32 : 16u, true);
     return decode_impl(view, NewRows{}, q, q_dtype, q_heads, scale, token_count, nullptr, nullptr, bound, out, gate,
                        gated_out, nullptr, workspace, workspace_bytes, stream, &rs);
 }

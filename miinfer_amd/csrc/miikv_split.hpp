@@ -17,9 +17,9 @@ struct SplitArgs {
     uint32_t q_heads;
     uint32_t group;  // columns per (row set, kv head), <= 16: pack tokens x query heads per kv head
     // Tokens per row set (1: decode).  A short suffix packs `pack` consecutive tokens of
-    // one sequence into a row set: column c is token pack*b + c / (group / pack), query
-    // head h * (group / pack) + c % (group / pack), with context split_length() - (pack -
-    // 1 - c / (group / pack)).
+    // one sequence into a row set: column c is token t = pack*b + c / (group / pack), query
+    // head h * (group / pack) + c % (group / pack), with t's context (host lengths, the last
+    // token's is max_context); the last row set's tokens past it are not stored.
     uint32_t pack;
     float scale_log2;
     // Context length of row-set b: (len_ptr ? len_ptr[b * len_stride] : 0) + len_add
@@ -166,6 +166,11 @@ __device__ __forceinline__ void stream_records(const SplitArgs& a, uint32_t b, u
     count = w1 - w0 + 1;
 }
 
+// Context of token tp of row set b of a packed suffix (past the suffix: above max_context).
+__device__ __forceinline__ uint32_t packed_context(const SplitArgs& a, uint32_t b, uint32_t tp) {
+    return a.len_add + b * a.len_bstep - (a.pack - 1 - tp);
+}
+
 // Split count of sequence b at `cpw` steps per wave (0 when L == 0).
 __device__ __forceinline__ uint32_t split_count(uint32_t L, uint32_t cpw) {
     const uint32_t tps = kWavesPerWg * cpw * kChunk;
@@ -305,6 +310,7 @@ __global__ void __launch_bounds__(256) combine_kernel(SplitArgs a) {
     // output row of column hn (packed tokens: token pack*b + hn / Gt, head h*Gt + hn % Gt),
     // indexed below with the column's offset e - hn * D folded back in
     const uint32_t Gt = G / a.pack, tp = hn / Gt;
+    if (a.pack > 1 && packed_context(a, b, tp) > a.max_context) return;  // past the suffix (workgroup-uniform)
     const size_t out_row0 = ((static_cast<size_t>(b) * a.pack + tp) * a.q_heads + static_cast<size_t>(h) * Gt +
                              (hn - tp * Gt)) * D - static_cast<size_t>(hn) * D;
     const uint32_t rec = record_floats(G, D);
@@ -381,16 +387,18 @@ __global__ void __launch_bounds__(256) combine_narrow_kernel(SplitArgs a) {
     const uint64_t idx = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
     const uint64_t per = GD / 4;
     const uint32_t bh = static_cast<uint32_t>(idx / per);
-    const bool live = bh < a.batch * a.g.kv_heads;
-    const uint32_t bhc = live ? bh : 0;
+    const bool row_live = bh < a.batch * a.g.kv_heads;
+    const uint32_t bhc = row_live ? bh : 0;
     const uint32_t b = bhc / a.g.kv_heads;
     const uint32_t h = bhc % a.g.kv_heads;
     const uint32_t e = static_cast<uint32_t>(idx % per) * 4;
     const uint32_t q = (e / 4) & 7;
     const uint32_t hn = e / D;
     const uint32_t Gt = G / a.pack, tp = hn / Gt;
-    const size_t out_row0 = ((static_cast<size_t>(b) * a.pack + tp) * a.q_heads + static_cast<size_t>(h) * Gt +
-                             (hn - tp * Gt)) * D - static_cast<size_t>(hn) * D;
+    const bool past = a.pack > 1 && packed_context(a, b, tp) > a.max_context;  // past the suffix: not stored
+    const bool live = row_live && !past;
+    const size_t out_row0 = ((static_cast<size_t>(b) * a.pack + (past ? 0u : tp)) * a.q_heads +
+                             static_cast<size_t>(h) * Gt + (hn - tp * Gt)) * D - static_cast<size_t>(hn) * D;
     const uint32_t rec = record_floats(G, D);
     const CombineRecords R = combine_records(a, b, h, bhc, APPEND);
     // The first batch of record slots is read before the context length arrives (slots

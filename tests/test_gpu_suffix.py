@@ -741,3 +741,31 @@ def test_suffix_workgroup_forms(gpu, hq, hk, d, prefix, t):
         s = q[:, h].double() @ k[h // (hq // hk)].T.contiguous() / math.sqrt(d)
         expect = torch.softmax(s.masked_fill(hidden, -math.inf), -1) @ v[h // (hq // hk)]
         assert_attention_close(out[:, h].cpu().numpy(), expect.cpu().numpy(), f"head {h}")
+
+
+@pytest.mark.parametrize("hq,hk,d,prefix,t", [(32, 8, 128, 3000, 5), (32, 8, 128, 40, 7), (24, 4, 256, 2000, 11),
+                                              (24, 4, 256, 61, 3), (32, 8, 128, 500, 10)])
+@pytest.mark.parametrize("f32", [False, True])
+def test_suffix_short_last_row_set_not_full(gpu, hq, hk, d, prefix, t, f32):
+    """Token counts that the packed columns do not divide: the last row set's unused columns
+    read no row past the query and store none, every token attends to its own context."""
+    import miinfer_amd as m
+    rng = np.random.default_rng(prefix + t)
+    n = prefix + t
+    cache = m.KvCache.contiguous(hk, d, (n + 63) // 64 * 64)
+    cache.append(_dev(randn_f16(rng, (n, hk, d)), gpu), _dev(randn_f16(rng, (n, hk, d)), gpu))
+    q = _dev(rng.standard_normal((t, hq, d)).astype(np.float32), gpu)
+    q = q if f32 else q.half()
+    room = torch.full((t + 4, hq, d), 7.0, device=gpu)
+    gated = torch.full((t + 4, hq, d), 7.0, device=gpu)
+    gate = _dev(rng.standard_normal((t, hq, d)).astype(np.float32), gpu)
+    m.suffix_attention(cache, q, prefix, out=room[:t], gate=gate, gated_out=gated[:t])
+    assert bool((room[t:] == 7.0).all()) and bool((gated[t:] == 7.0).all())
+    k, v = (x.double() for x in cache.export_dequant(0, 0, n))
+    hidden = torch.arange(n, device=gpu)[None, :] > prefix + torch.arange(t, device=gpu)[:, None]
+    for h in range(hq):
+        s = q[:, h].double() @ k[h // (hq // hk)].T.contiguous() / math.sqrt(d)
+        expect = torch.softmax(s.masked_fill(hidden, -math.inf), -1) @ v[h // (hq // hk)]
+        assert_attention_close(room[:t, h].cpu().numpy(), expect.cpu().numpy(), f"head {h}")
+        assert_attention_close(gated[:t, h].cpu().numpy(), (expect * torch.sigmoid(gate[:, h].double())).cpu().numpy(),
+                               f"gated head {h}")
