@@ -32,6 +32,7 @@
 #include "miikv_common.hpp"
 #include "miikv_split.hpp"
 
+#include <array>
 #include <cmath>
 #include <cstdlib>
 #include <mutex>
@@ -984,6 +985,12 @@ struct Plan {
     uint64_t part_bytes;
 };
 
+// D = 256, one sequence: a wave holds one step in flight (its step buffer is twice D =
+// 128's), and one workgroup per CU with twice the steps per wave measured faster than two
+// (24q/4kv batch 1, µs: 16k 17.9 -> 16.7, 32k 24.1 -> 23.0; 4k and 64k unchanged).  Batches
+// keep the full target (config 3 is tuned so).
+uint64_t target_waves(uint32_t D, uint32_t batch) { return D == 256 && batch == 1 ? kTargetWaves / 2 : kTargetWaves; }
+
 // rowsets: row sets of one sequence (a suffix run as decodes), all of about the same
 // length: XCD-ordered.  They all read the same keys: with long items the workgroups
 // running at once stream the same addresses together, so the steps per wave are capped
@@ -993,11 +1000,7 @@ Plan make_plan(const miikv_view* v, uint32_t q_heads, uint32_t batch, uint32_t m
     Plan p;
     const uint64_t chunks = (static_cast<uint64_t>(max_context) + kChunk - 1) / kChunk;
     const uint64_t waves = chunks * v->kv_heads * batch;
-    // D = 256, one sequence: a wave holds one step in flight (its step buffer is
-    // twice D = 128's), and one workgroup per CU with twice the steps per wave
-    // measured faster than two (24q/4kv batch 1, µs: 16k 17.9 -> 16.7, 32k 24.1 ->
-    // 23.0; 4k and 64k unchanged).  Batches keep the full target (config 3 is tuned so).
-    const uint64_t target = (v->head_dim == 256 && batch == 1) ? kTargetWaves / 2 : kTargetWaves;
+    const uint64_t target = target_waves(v->head_dim, batch);
     uint64_t cpw = (waves + target - 1) / target;
     // A batch: records for splits of a quarter of the all-sequences-full value, which the
     // streamed plan (stream_workgroups) shares out.
@@ -1339,14 +1342,42 @@ uint32_t suffix_pack(const miikv_view* view, uint32_t q_heads, uint32_t token_co
     return 1;
 }
 
+// Every packing a suffix may run with: unpacked (device count), even and ragged, of fp16
+// and fp32 queries.
+static std::array<uint32_t, 5> suffix_packs(const miikv_view* view, uint32_t q_heads, uint32_t token_count) {
+    return {1u, suffix_pack(view, q_heads, token_count, false, 16, false),
+            suffix_pack(view, q_heads, token_count, false, kRowsetColsF32, false),
+            suffix_pack(view, q_heads, token_count, false, 16, true),
+            suffix_pack(view, q_heads, token_count, false, kRowsetColsF32, true)};
+}
+
+static uint64_t rowset_bytes(const miikv_view* view, uint32_t q_heads, uint32_t token_count, uint32_t pack, uint32_t bound) {
+    const Plan p = make_plan(view, q_heads * pack, (token_count + pack - 1) / pack, bound, kRowsetMaxCpw, true);
+    return p.counter_bytes + p.part_bytes;
+}
+
 uint64_t suffix_by_decode_bytes(const miikv_view* view, uint32_t q_heads, uint32_t token_count, uint32_t bound) {
-    // the largest of the packed plans (fp16 and fp32 queries, host token count) and the
-    // unpacked one (device count)
+    // with the evenly packed plans the route is open; a ragged one is taken where its own
+    // records fit too (suffix_by_decode)
     uint64_t most = 0;
-    for (const uint32_t pk : {1u, suffix_pack(view, q_heads, token_count, false, 16, true),
-                              suffix_pack(view, q_heads, token_count, false, kRowsetColsF32, true)}) {
-        const Plan p = make_plan(view, q_heads * pk, (token_count + pk - 1) / pk, bound, kRowsetMaxCpw, true);
-        most = std::max(most, p.counter_bytes + p.part_bytes);
+    const auto packs = suffix_packs(view, q_heads, token_count);
+    for (uint32_t i = 0; i < 3; ++i) most = std::max(most, rowset_bytes(view, q_heads, token_count, packs[i], bound));
+    return most;
+}
+
+// Records are not monotone in the context: where the steps per wave go up by one, the splits
+// drop.  Within one count of steps they are, so the most that any context up to `bound`
+// takes is at `bound` or at the longest context of a smaller count.
+uint64_t suffix_by_decode_bytes_up_to(const miikv_view* view, uint32_t q_heads, uint32_t token_count, uint32_t bound) {
+    uint64_t most = 0;
+    for (const uint32_t pk : suffix_packs(view, q_heads, token_count)) {
+        const uint32_t sets = (token_count + pk - 1) / pk;
+        const Plan at_bound = make_plan(view, q_heads * pk, sets, bound, kRowsetMaxCpw, true);
+        most = std::max(most, at_bound.counter_bytes + at_bound.part_bytes);
+        for (uint32_t cpw = 1; cpw < at_bound.cpw; ++cpw) {
+            const uint64_t keys = cpw * target_waves(view->head_dim, sets) / (static_cast<uint64_t>(view->kv_heads) * sets) * kChunk;
+            if (keys != 0 && keys < bound) most = std::max(most, rowset_bytes(view, q_heads, token_count, pk, static_cast<uint32_t>(keys)));
+        }
     }
     return most;
 }
@@ -1366,7 +1397,10 @@ miikv_status suffix_by_decode(const miikv_view* view, const void* q, uint32_t q_
     // fragment set (T = 2: 16.6 against 17.2 us; the exact route at T = 512: 790
     // against 963 us, where twice the row sets' operand conversions cost more).
     const bool pair_cols = q_dtype == MIIKV_DTYPE_F32 && token_count >= 4 && token_count <= 16;
-    rs.pack = suffix_pack(view, q_heads, token_count, prefill_state != nullptr, pair_cols ? kRowsetColsF32 : 16u, true);
+    const uint32_t cols = pair_cols ? kRowsetColsF32 : 16u;
+    rs.pack = suffix_pack(view, q_heads, token_count, prefill_state != nullptr, cols, true);
+    if (workspace_bytes < rowset_bytes(view, q_heads, token_count, rs.pack, bound))
+        rs.pack = suffix_pack(view, q_heads, token_count, prefill_state != nullptr, cols, false);
     return decode_impl(view, NewRows{}, q, q_dtype, q_heads, scale, token_count, nullptr, nullptr, bound, out, gate,
                        gated_out, nullptr, workspace, workspace_bytes, stream, &rs);
 }

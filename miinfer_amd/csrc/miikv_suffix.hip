@@ -1197,7 +1197,7 @@ extern "C" uint64_t miikv_suffix_workspace_bytes(const miikv_view* view, uint32_
     uint64_t dec = 0;
     if (suffix_runs_as_decode(view, q_heads, token_count, false) ||
         suffix_runs_as_decode(view, q_heads, token_count, true))
-        dec = suffix_by_decode_bytes(view, q_heads, token_count, static_cast<uint32_t>(std::min<uint64_t>(cap, 0xffffffffu)));
+        dec = suffix_by_decode_bytes_up_to(view, q_heads, token_count, static_cast<uint32_t>(std::min<uint64_t>(cap, 0xffffffffu)));
     const SuffixPlan p = make_suffix_plan(view, q_heads, token_count, cap, true);
     // (the 4-wave form splits only where the 8-wave form does)
     const SuffixPlan small = make_suffix_plan(view, q_heads, token_count, cap, p.splits > 1, 0, false, kSufWavesSmall);
@@ -1216,7 +1216,7 @@ extern "C" uint64_t miikv_suffix_workspace_bytes_ex(const miikv_view* view, uint
     const SuffixPlan tiles = make_suffix_plan(view, q_heads, token_count, cap, false);
     const uint32_t cap32 = static_cast<uint32_t>(std::min<uint64_t>(cap, 0xffffffffu));
     const SuffixPlan xp = make_suffix_plan(view, q_heads, token_count, cap, true, 0, true);
-    return std::max({base, tiles.tile_bytes + suffix_by_decode_bytes(view, q_heads, token_count, cap32),
+    return std::max({base, tiles.tile_bytes + suffix_by_decode_bytes_up_to(view, q_heads, token_count, cap32),
                      xp.total()});
 }
 

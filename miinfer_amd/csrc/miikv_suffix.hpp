@@ -27,7 +27,10 @@ constexpr uint32_t kSuffixDecodeMaxT = 64;
 uint32_t suffix_pack(const miikv_view* view, uint32_t q_heads, uint32_t token_count, bool device_count,
                      uint32_t max_cols = 16, bool ragged = false);
 bool decode_columns_fit(uint32_t G, uint32_t D);  // decode_kernel serves G columns at head_dim D
+// Workspace with which a suffix of at most `bound` keys runs as decodes; and the most that any
+// context up to `bound` can use.
 uint64_t suffix_by_decode_bytes(const miikv_view* view, uint32_t q_heads, uint32_t token_count, uint32_t bound);
+uint64_t suffix_by_decode_bytes_up_to(const miikv_view* view, uint32_t q_heads, uint32_t token_count, uint32_t bound);
 miikv_status suffix_by_decode(const miikv_view* view, const void* q, uint32_t q_dtype, uint32_t q_heads, float scale,
                               uint32_t token_count, uint32_t base_position, uint32_t seq,
                               const miikv_prefill_state* prefill_state, uint32_t bound, float* out, const float* gate,

@@ -217,3 +217,24 @@ def test_suffix_workspace_bytes_ex():
     wide = _view(page_tokens=1024, kv_heads=1, head_dim=128)
     assert lib.miikv_suffix_workspace_bytes_ex(ctypes.byref(wide), 32, 64, L.SUFFIX_EXACT) == 0  # 32 heads per kv head
     assert lib.miikv_suffix_workspace_bytes_ex(ctypes.byref(wide), 32, 64, 0) > 0
+
+
+@pytest.mark.parametrize("hq,hk,d", [(32, 8, 128), (24, 4, 256)])
+@pytest.mark.parametrize("tokens", [2, 3, 4, 5, 7, 8, 11, 12, 40])
+def test_suffix_workspace_bytes_ex_serves_every_base_position(hq, hk, d, tokens):
+    """The queried size is enough wherever the suffix starts: the records of a shorter context
+    can be more than the capacity's (they drop where the steps per wave go up by one)."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("the accepted calls would launch on made-up addresses")
+    L = _lib()
+    lib = L.lib()
+    p = ctypes.c_void_p(0x10000)
+    flags = L.SUFFIX_TILES_CURRENT | L.SUFFIX_EXACT
+    for cap in (640, 1088, 2112, 4224, 5568, 8320, 16384, 20032):
+        v = _view(page_tokens=cap, kv_heads=hk, head_dim=d)
+        need = lib.miikv_suffix_workspace_bytes_ex(ctypes.byref(v), hq, tokens, flags)
+        for base in range(0, cap - tokens + 1, 31):
+            st = lib.miikv_suffix_attn_ex(ctypes.byref(v), None, None, p, L.DTYPE_F16, hq, 0.1, tokens, base, 0, None,
+                                          flags, p, None, None, p, need, None)
+            assert st != L.MIIKV_EWORKSPACE, (cap, base)

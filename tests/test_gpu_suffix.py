@@ -769,3 +769,37 @@ def test_suffix_short_last_row_set_not_full(gpu, hq, hk, d, prefix, t, f32):
         assert_attention_close(room[:t, h].cpu().numpy(), expect.cpu().numpy(), f"head {h}")
         assert_attention_close(gated[:t, h].cpu().numpy(), (expect * torch.sigmoid(gate[:, h].double())).cpu().numpy(),
                                f"gated head {h}")
+
+
+@pytest.mark.parametrize("hq,hk,d", [(32, 8, 128), (24, 4, 256)])
+def test_suffix_exact_at_every_accepted_workspace_size(gpu, hq, hk, d):
+    """A short exact suffix in workspaces from the queried size down: the packing whose records
+    do not fit gives way to the even one, and no call writes past the size it was given."""
+    import miinfer_amd as m
+    from miinfer_amd import _lib
+    prefix, t = 2900, 5
+    rng = np.random.default_rng(t)
+    n = prefix + t
+    cache = m.KvCache.contiguous(hk, d, 4224)
+    cache.append(_dev(randn_f16(rng, (n, hk, d)), gpu), _dev(randn_f16(rng, (n, hk, d)), gpu))
+    q = _dev(randn_f16(rng, (t, hq, d)), gpu)
+    need = m.suffix_workspace_bytes(cache, hq, t, exact=True)
+    buf = torch.empty(need + 4096, dtype=torch.uint8, device=gpu)
+    k, v = (x.double() for x in cache.export_dequant(0, 0, n))
+    hidden = torch.arange(n, device=gpu)[None, :] > prefix + torch.arange(t, device=gpu)[:, None]
+    sizes = sorted({need, *(int(need * f) // 256 * 256 for f in np.linspace(0.02, 1.0, 50))}, reverse=True)
+    ran = 0
+    for size in sizes:
+        buf[size:].fill_(0x5A)
+        try:
+            out, _ = m.suffix_attention(cache, q, prefix, exact=True, workspace=buf[:size])
+        except _lib.MiikvError as e:
+            assert e.status == _lib.MIIKV_EWORKSPACE
+            break
+        ran += 1
+        assert bool((buf[size:] == 0x5A).all())
+        for h in range(hq):
+            s = q[:, h].double() @ k[h // (hq // hk)].T.contiguous() / math.sqrt(d)
+            expect = torch.softmax(s.masked_fill(hidden, -math.inf), -1) @ v[h // (hq // hk)]
+            assert_attention_close(out[:, h].cpu().numpy(), expect.cpu().numpy(), f"{size} bytes head {h}")
+    assert ran > 2
