@@ -251,69 +251,79 @@ __global__ void __launch_bounds__(256) append_kernel(
 // each kind.  The partial groups at either end of the rows store theirs token by token, in
 // the same launch.  Every token lies inside the sequence's capacity (checked on the host).
 // Bound: HBM, given three workgroups per CU (at two, 21.6 us below).  8195 fp32 rows with
-// the K prologue at position 77, 4 kv heads, D = 256 (85 MB): 34.2 -> 19.6 us (4.3 TB/s);
+// the K prologue at position 77, 4 kv heads, D = 256 (85 MB): 34.2 -> 20.0 us (4.3 TB/s);
 // launches of their own for the partial groups took 13 of it.  4096 fp16 rows at position
-// 5, 8 kv heads, D = 128: 16.6 -> 8.8; whole groups alone (8192 fp16 rows at 0) 10.0 -> 10.3.
-template <bool F32>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) append_tile_kernel(Geo g, AppendIn in, uint32_t token_count,
-                                                          uint32_t base_position, uint32_t seq) {
+// 5, 8 kv heads, D = 128: 15.3 -> 6.6.
+// Instances with and without the prologue (NORM) and partial groups (PARTIAL): with both in
+// one kernel the rows that need neither paid 0.1 - 0.3 us for them (64 fp32 rows without the
+// prologue, 8 kv heads, D = 128 3.13 -> 3.39; now 3.02; 64 fp16 rows 2.91 -> 3.04 -> 2.91).
+template <bool F32, bool NORM, bool PARTIAL>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NORM ? 6 : 2))) append_tile_kernel(
+    Geo g, AppendIn in, uint32_t base_position, uint32_t seq, uint32_t token_count) {
+    static_assert(F32 || !NORM, "the K prologue takes fp32 rows");
     extern __shared__ uint4 s_tile[];
     const uint32_t D = g.head_dim;
     const uint32_t groups = D / 16;
     const uint32_t head = blockIdx.y;
     const uint32_t tl = threadIdx.x / groups;  // token within the 32-token group
     const uint32_t q16 = threadIdx.x % groups;
-    const uint32_t pos0 = (base_position / 32 + blockIdx.x) * 32;  // the group's first position
+    // the group's first position
+    const uint32_t pos0 = PARTIAL ? (base_position / 32 + blockIdx.x) * 32 : base_position + blockIdx.x * 32;
     const uint32_t pos = pos0 + tl;
-    const bool mine = pos >= base_position && pos - base_position < token_count;
-    const uint32_t token = mine ? pos - base_position : 0;  // others compute a row and drop it
+    const bool mine = !PARTIAL || (pos >= base_position && pos - base_position < token_count);
+    // (others compute a row and drop it)
+    const uint32_t token = !PARTIAL ? blockIdx.x * 32 + tl : mine ? pos - base_position : 0;
     const size_t src = (static_cast<size_t>(token) * g.kv_heads + head) * D + q16 * 16;
     float xk[16], xv[16];
-    if constexpr (F32) {
+    if constexpr (NORM) {
         load16_f32(static_cast<const float*>(in.v) + src, xv);
         load16_f32(static_cast<const float*>(in.k) + src, xk);
+    } else if constexpr (F32) {
+        load16_f32(static_cast<const float*>(in.k) + src, xk);
+        load16_f32(static_cast<const float*>(in.v) + src, xv);
+        // Every load ahead of the first wait.  Left to itself the compiler waits for K before
+        // it loads V: 8192 rows, 8 kv heads, D = 128 15.9 us against 14.0.
+        __builtin_amdgcn_sched_barrier(0);
     } else {
-        load16_f16(static_cast<const uint16_t*>(in.v) + src, xv);
         load16_f16(static_cast<const uint16_t*>(in.k) + src, xk);
+        load16_f16(static_cast<const uint16_t*>(in.v) + src, xv);
     }
-    // V first: packed, its values leave their registers before K's prologue
     uint4 vpk, kpk;
     float sk, sv;
-    {
-        int8_t q[16];
-        quantize16(xv, q, sv);
-        vpk = pack16_codes(q);
-    }
-    if constexpr (F32) {
-        if (in.k_norm_weight != nullptr) {
-            // The rotations of the group's 32 tokens, shared out over all threads (a rotating
-            // lane computing its own 16 keeps three quarters of the lanes idle meanwhile).
-            __shared__ float2 s_rot[32][33];  // [token][pair] (sine, cosine)
-            auto prologue = [&](auto tag) __attribute__((always_inline)) {
-                constexpr uint32_t GROUPS = decltype(tag)::value, PER = 32 / GROUPS;
-                float angle = rope_angle<31>(pos, in.rope_step, PER * q16);
+    int8_t qk[16], qv[16];
+    if constexpr (NORM) {
+        // V first: packed, its values leave their registers before K's prologue
+        quantize16(xv, qv, sv);
+        vpk = pack16_codes(qv);
+        // The rotations of the group's 32 tokens, shared out over all threads (a rotating
+        // lane computing its own 16 keeps three quarters of the lanes idle meanwhile).
+        __shared__ float2 s_rot[32][33];  // [token][pair] (sine, cosine)
+        auto prologue = [&](auto tag) __attribute__((always_inline)) {
+            constexpr uint32_t GROUPS = decltype(tag)::value, PER = 32 / GROUPS;
+            float angle = rope_angle<31>(pos, in.rope_step, PER * q16);
 #pragma unroll
-                for (uint32_t k = 0; k < PER; ++k) {
-                    float2 sc;
-                    rope_sincos(angle, &sc.x, &sc.y);
-                    s_rot[tl][PER * q16 + k] = sc;
-                    angle *= in.rope_step;
-                }
-                // written and read by the same wave (a token's lanes): no barrier
-                const float2* rot = &s_rot[tl][16 * (q16 & 1)];
-                k_norm_rope16<GROUPS>(xk, in.k_norm_weight, q16, in.epsilon,
-                                      [&](int j) __attribute__((always_inline)) { return rot[j]; });
-            };
-            if (groups == 16) prologue(std::integral_constant<uint32_t, 16>{});
-            else prologue(std::integral_constant<uint32_t, 8>{});
-        }
+            for (uint32_t k = 0; k < PER; ++k) {
+                float2 sc;
+                rope_sincos(angle, &sc.x, &sc.y);
+                s_rot[tl][PER * q16 + k] = sc;
+                angle *= in.rope_step;
+            }
+            // written and read by the same wave (a token's lanes): no barrier
+            const float2* rot = &s_rot[tl][16 * (q16 & 1)];
+            k_norm_rope16<GROUPS>(xk, in.k_norm_weight, q16, in.epsilon,
+                                  [&](int j) __attribute__((always_inline)) { return rot[j]; });
+        };
+        if (groups == 16) prologue(std::integral_constant<uint32_t, 16>{});
+        else prologue(std::integral_constant<uint32_t, 8>{});
+        quantize16(xk, qk, sk);
+        kpk = pack16_codes(qk);
+    } else {
+        quantize16(xk, qk, sk);
+        quantize16(xv, qv, sv);
+        kpk = pack16_codes(qk);
+        vpk = pack16_codes(qv);
     }
-    {
-        int8_t q[16];
-        quantize16(xk, q, sk);
-        kpk = pack16_codes(q);
-    }
-    if (pos0 < base_position || pos0 + 31 - base_position >= token_count) {  // a partial group (workgroup-uniform)
+    if (PARTIAL && (pos0 < base_position || pos0 + 31 - base_position >= token_count)) {  // a partial group (workgroup-uniform)
         if (mine) {
             const size_t slab = slab_of(g, seq, pos, head);
             store_k_codes16(g, slab, pos % g.page_tokens, q16, kpk, sk);
@@ -342,28 +352,29 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) a
     const size_t slab_bytes = static_cast<size_t>(g.page_tokens) * D;
     uint4* kdst = reinterpret_cast<uint4*>(g.k_codes + slab * slab_bytes + static_cast<size_t>(tp0) * D);
     uint4* vdst = reinterpret_cast<uint4*>(g.v_codes + slab * slab_bytes + static_cast<size_t>(tp0) * D);
-    const uint32_t chunks = 32 * D / 16;  // 16-byte chunks per code region
-    for (uint32_t c = threadIdx.x; c < chunks; c += blockDim.x) {
-        kdst[c] = s_tile[c];
-        // V chunk c: dim d = c/2, slab bytes 16*(c%2) .. +15 of that dim hold tokens
-        // 16J + 4G + I at 8G + 4J + I, G = 2*(c%2) + {0, 1}: four 4-token runs.
-        const uint32_t d = c / 2, g0 = 2 * (c % 2);
-        uint32_t w[4];
+    // 16-byte chunks per code region: as many as there are threads, one each (asking for the
+    // workgroup's size instead reads another line of kernel arguments: 0.08 us)
+    const uint32_t chunks = 32 * D / 16;
+    const uint32_t c = threadIdx.x;
+    kdst[c] = s_tile[c];
+    // V chunk c: dim d = c/2, slab bytes 16*(c%2) .. +15 of that dim hold tokens
+    // 16J + 4G + I at 8G + 4J + I, G = 2*(c%2) + {0, 1}: four 4-token runs.
+    const uint32_t d = c / 2, g0 = 2 * (c % 2);
+    uint32_t w[4];
 #pragma unroll
-        for (uint32_t k = 0; k < 4; ++k) {
-            const uint32_t t0 = 16 * (k % 2) + 4 * (g0 + k / 2);
-            w[k] = static_cast<uint32_t>(s_v[t0 * D + d]) | (static_cast<uint32_t>(s_v[(t0 + 1) * D + d]) << 8) |
-                   (static_cast<uint32_t>(s_v[(t0 + 2) * D + d]) << 16) |
-                   (static_cast<uint32_t>(s_v[(t0 + 3) * D + d]) << 24);
-        }
-        vdst[c] = make_uint4(w[0], w[1], w[2], w[3]);
+    for (uint32_t k = 0; k < 4; ++k) {
+        const uint32_t t0 = 16 * (k % 2) + 4 * (g0 + k / 2);
+        w[k] = static_cast<uint32_t>(s_v[t0 * D + d]) | (static_cast<uint32_t>(s_v[(t0 + 1) * D + d]) << 8) |
+               (static_cast<uint32_t>(s_v[(t0 + 2) * D + d]) << 16) |
+               (static_cast<uint32_t>(s_v[(t0 + 3) * D + d]) << 24);
     }
+    vdst[c] = make_uint4(w[0], w[1], w[2], w[3]);
     const uint32_t schunks = 32 * (D / 32) * 2 / 16;  // 16-byte chunks per scale region
     const size_t sidx = (slab * g.page_tokens + tp0) * (D / 32);
     if (threadIdx.x < 2 * schunks) {
-        const uint32_t kind = threadIdx.x / schunks, c = threadIdx.x % schunks;
+        const uint32_t kind = threadIdx.x / schunks, sc = threadIdx.x % schunks;
         uint16_t* sdst = (kind == 0 ? g.k_scales : g.v_scales) + sidx;
-        reinterpret_cast<uint4*>(sdst)[c] = s_tile[2 * chunks + kind * schunks + c];
+        reinterpret_cast<uint4*>(sdst)[sc] = s_tile[2 * chunks + kind * schunks + sc];
     }
 }
 
@@ -701,9 +712,20 @@ static miikv_status launch_append(const miikv_view* view, const AppendIn& in, ui
         const uint32_t D = view->head_dim;
         const uint64_t groups = (static_cast<uint64_t>(base) + rows_tokens + 31) / 32 - base / 32;
         const size_t lds = 2 * 32 * D + 2 * 32 * (D / 32) * sizeof(uint16_t);
-        hipLaunchKernelGGL(append_tile_kernel<F32>, dim3(static_cast<uint32_t>(groups), view->kv_heads),
-                           dim3(32 * (D / 16)), lds, static_cast<hipStream_t>(stream), make_geo(*view), in,
-                           rows_tokens, base, seq);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(groups), view->kv_heads), dim3(32 * (D / 16)), lds,
+                               static_cast<hipStream_t>(stream), make_geo(*view), in, base, seq, rows_tokens);
+        };
+        const bool partial = base % 32 != 0 || rows_tokens % 32 != 0;
+        if constexpr (F32) {
+            if (in.k_norm_weight != nullptr) {
+                if (partial) launch(append_tile_kernel<true, true, true>);
+                else launch(append_tile_kernel<true, true, false>);
+                return launch_status();
+            }
+        }
+        if (partial) launch(append_tile_kernel<F32, false, true>);
+        else launch(append_tile_kernel<F32, false, false>);
         return launch_status();
     }
     return launch_rows<F32>(view, in, rows_tokens, base, seq, ps, ds, positions, stream);

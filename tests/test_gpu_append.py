@@ -277,3 +277,25 @@ def test_append_bulk_ends_inside_groups(gpu, base, t):
     for i, x in enumerate(rows):
         codes, scales = oracle.quantize_rows(x.transpose(1, 0, 2))
         assert np.array_equal(got[2 * i], codes) and np.array_equal(got[2 * i + 1], scales)
+
+
+@pytest.mark.parametrize("base,t", [(0, 64), (32, 96), (5, 70), (0, 65), (27, 101)])
+@pytest.mark.parametrize("kind", ["f16", "f32", "norm"])
+@pytest.mark.parametrize("hk,d", [(3, 128), (2, 256)])
+def test_append_bulk_equals_short_appends(gpu, hk, d, kind, base, t):
+    """Each form of the bulk append (fp16 rows, fp32 rows with and without the K prologue, whole
+    and partial groups) stores the bytes of appends too short for it."""
+    import miinfer_amd as m
+    rng = np.random.default_rng(base + t)
+    k, v = (_dev(rng.standard_normal((t, hk, d)).astype(np.float32), gpu) for _ in range(2))
+    w = _dev(rng.uniform(0.5, 1.5, d).astype(np.float32), gpu) if kind == "norm" else None
+    caches = [m.KvCache.contiguous(hk, d, 192) for _ in range(2)]
+    for c, step in zip(caches, (t, 31)):
+        for i in range(0, t, step):
+            rows = [x[i:i + step] for x in (k, v)]
+            if kind == "f16":
+                c.append(*(x.half() for x in rows), base_position=base + i)
+            else:
+                c.append_f32(*rows, base + i, k_norm_weight=w)
+    for a, b in zip(*((c.k_codes, c.k_scales, c.v_codes, c.v_scales) for c in caches)):
+        assert torch.equal(a, b)
