@@ -212,7 +212,7 @@ __device__ void k_prologue(float& kx, float w, uint32_t tid, uint32_t position, 
 // heads, and write the token's record (m = score, l = 1, O = dequantised V row for
 // every head) at slot nsplit, after the splits, which cover the L-1 cached keys.
 // The row and query loads go out before the context length arrives.
-template <uint32_t D>
+template <uint32_t D, bool STREAM>
 __device__ void append_record(const SplitArgs& a, uint32_t b, uint32_t h) {
     constexpr uint32_t DJ = D / 64;
     __shared__ float s_k[D];
@@ -280,7 +280,7 @@ __device__ void append_record(const SplitArgs& a, uint32_t b, uint32_t h) {
     __syncthreads();
     const uint32_t rec = record_floats(G, D);
     const size_t bh = static_cast<size_t>(b) * a.g.kv_heads + h;
-    const size_t slot = a.stream_wgs != 0 ? static_cast<size_t>(a.batch) * a.g.kv_heads * a.max_splits + bh
+    const size_t slot = STREAM ? static_cast<size_t>(a.batch) * a.g.kv_heads * a.max_splits + bh
                                           : bh * (a.max_splits + 1) + split_count(L, a.cpw);
     float* r = a.part + slot * rec;
     for (uint32_t i4 = tid; i4 < G * D / 4; i4 += 256) {
@@ -357,7 +357,7 @@ decode_kernel(SplitArgs a) {
         if (blockIdx.x >= first) {
             const uint32_t x = blockIdx.x - first;
             const uint32_t ab = x / a.g.kv_heads;
-            if (a.count_ptr == nullptr || ab < *a.count_ptr) append_record<D>(a, ab, x % a.g.kv_heads);
+            if (a.count_ptr == nullptr || ab < *a.count_ptr) append_record<D, STREAM>(a, ab, x % a.g.kv_heads);
             return;
         }
     }
@@ -836,7 +836,7 @@ decode_kernel(SplitArgs a) {
 
     // Partial record of one run: [O: G*D][m: G][l: G] padded to a multiple of 4 floats,
     // so every record starts 16-byte aligned.
-    for (uint32_t c4 = tid; c4 < G * D / 4; c4 += blockDim.x) {
+    for (uint32_t c4 = tid; c4 < G * D / 4; c4 += 64 * kWavesPerWg) {
         const uint32_t hn = (4 * c4) / D, dim = (4 * c4) % D;
         const uint32_t mt = dim / 16, gq = (dim % 16) / 4;
         float mw[kWavesPerWg];
@@ -949,8 +949,8 @@ decode_kernel(SplitArgs a) {
         } else {
             const uint32_t bh = blockIdx.x / a.max_splits;
             split = blockIdx.x % a.max_splits;
-            b = bh / geo.kv_heads;
-            h = bh % geo.kv_heads;
+            b = a.batch == 1 ? 0u : bh / geo.kv_heads;
+            h = bh - b * geo.kv_heads;
         }
         // Steps this wave may own, from the host bound alone: the first loads are issued
         // before the context length arrives from memory.
@@ -1295,19 +1295,24 @@ static miikv_status decode_impl(const miikv_view* view, const NewRows& rows,
     const dim3 ngrid(static_cast<uint32_t>((nthreads + 255) / 256));
     const bool app = rows.any();
     const bool kf = mode_k_f16(view->quant_mode), vf = mode_v_f16(view->quant_mode);
-    if (view->head_dim == 128) {
-        launch_decode<128>(f32, app, kf, vf, grid, lds, s, a);
-        if (narrow && app) hipLaunchKernelGGL((combine_narrow_kernel<128, true>), ngrid, dim3(256), 0, s, a);
-        else if (narrow) hipLaunchKernelGGL((combine_narrow_kernel<128, false>), ngrid, dim3(256), 0, s, a);
-        else if (app) hipLaunchKernelGGL((combine_kernel<128, true>), cgrid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((combine_kernel<128, false>), cgrid, dim3(256), 0, s, a);
-    } else {
-        launch_decode<256>(f32, app, kf, vf, grid, lds, s, a);
-        if (narrow && app) hipLaunchKernelGGL((combine_narrow_kernel<256, true>), ngrid, dim3(256), 0, s, a);
-        else if (narrow) hipLaunchKernelGGL((combine_narrow_kernel<256, false>), ngrid, dim3(256), 0, s, a);
-        else if (app) hipLaunchKernelGGL((combine_kernel<256, true>), cgrid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((combine_kernel<256, false>), cgrid, dim3(256), 0, s, a);
-    }
+    if (view->head_dim == 128) launch_decode<128>(f32, app, kf, vf, grid, lds, s, a);
+    else launch_decode<256>(f32, app, kf, vf, grid, lds, s, a);
+    const auto combine = [&](auto d, auto with_append, auto streamed) {
+        constexpr uint32_t D = decltype(d)::value;
+        constexpr bool APP = decltype(with_append)::value, STREAM = decltype(streamed)::value;
+        if (narrow) hipLaunchKernelGGL((combine_narrow_kernel<D, APP, STREAM>), ngrid, dim3(256), 0, s, a);
+        else hipLaunchKernelGGL((combine_kernel<D, APP, STREAM>), cgrid, dim3(256), 0, s, a);
+    };
+    const auto with_stream = [&](auto d, auto with_append) {
+        if (a.stream_wgs != 0) combine(d, with_append, std::true_type{});
+        else combine(d, with_append, std::false_type{});
+    };
+    const auto with_dim = [&](auto with_append) {
+        if (view->head_dim == 128) with_stream(std::integral_constant<uint32_t, 128>{}, with_append);
+        else with_stream(std::integral_constant<uint32_t, 256>{}, with_append);
+    };
+    if (app) with_dim(std::true_type{});
+    else with_dim(std::false_type{});
     return hip_status(hipGetLastError());
 }
 

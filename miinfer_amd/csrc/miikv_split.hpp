@@ -205,36 +205,40 @@ __device__ __forceinline__ void merge_state(float& m, float& l, float4& acc, flo
     acc.w = acc.w * f1 + a2.w * f2;
 }
 
-// Record slots of one (sequence b, kv head h): `first` on, and how many may be read before
-// the count is known.  Streamed plan: the segments' records, then the new token's.
+// Records of one (sequence b, kv head h), and how many may be read before the count is
+// known.  STREAM: the segments' records, then the new token's; otherwise all of the pair's
+// slots.  (Two instances: choosing at run time cost one sequence's decode 0.1 us.)
+template <bool STREAM>
 struct CombineRecords {
-    size_t first;
-    size_t appended;   // streamed plan: slot of the new token's record
-    uint32_t nseg;     // streamed plan: segments (the other plan: all slots)
+    const float* part;      // the first record
+    const float* appended;  // STREAM: the new token's record
+    uint32_t nseg;          // STREAM: segments
     uint32_t slots;
-    __device__ __forceinline__ const float* at(const SplitArgs& a, uint32_t j, uint32_t rec) const {
-        return a.part + (j < nseg ? first + j : appended) * rec;
+    __device__ __forceinline__ const float* at(uint32_t j, uint32_t rec) const {
+        if constexpr (STREAM) return j < nseg ? part + static_cast<size_t>(j) * rec : appended;
+        else return part + static_cast<size_t>(j) * rec;
     }
 };
-__device__ __forceinline__ CombineRecords combine_records(const SplitArgs& a, uint32_t b, uint32_t h, uint32_t bh,
-                                                          bool append) {
-    CombineRecords r;
-    if (a.stream_wgs == 0) {
-        r.nseg = r.slots = a.max_splits + 1;
-        r.first = static_cast<size_t>(bh) * r.slots;
-        r.appended = r.first;
-        return r;
+template <bool STREAM>
+__device__ __forceinline__ CombineRecords<STREAM> combine_records(const SplitArgs& a, uint32_t b, uint32_t h, uint32_t bh,
+                                                                  uint32_t rec, bool append) {
+    CombineRecords<STREAM> r;
+    if constexpr (STREAM) {
+        uint32_t first;
+        stream_records(a, b, h, append ? 1u : 0u, first, r.nseg);
+        r.part = a.part + static_cast<size_t>(first) * rec;
+        r.appended = a.part + (static_cast<size_t>(a.batch) * a.g.kv_heads * a.max_splits + bh) * rec;
+        r.slots = r.nseg + (append && split_length(a, b) > 0 ? 1u : 0u);
+    } else {
+        r.slots = a.max_splits + 1;
+        r.part = a.part + (static_cast<size_t>(bh) * r.slots) * rec;
     }
-    uint32_t first;
-    stream_records(a, b, h, append ? 1u : 0u, first, r.nseg);
-    r.first = first;
-    r.appended = static_cast<size_t>(a.batch) * a.g.kv_heads * a.max_splits + bh;
-    r.slots = r.nseg + (append && split_length(a, b) > 0 ? 1u : 0u);
     return r;
 }
 // Records of sequence b (the plan of fixed splits waits for its length here).
-__device__ __forceinline__ uint32_t combine_count(const SplitArgs& a, uint32_t b, const CombineRecords& r, bool append) {
-    if (a.stream_wgs != 0) return r.slots;
+template <bool STREAM>
+__device__ __forceinline__ uint32_t combine_count(const SplitArgs& a, uint32_t b, const CombineRecords<STREAM>& r, bool append) {
+    if constexpr (STREAM) return r.slots;
     const uint32_t L = split_length(a, b);
     return split_count(L, a.cpw) + (append && L > 0 ? 1u : 0u);
 }
@@ -296,7 +300,7 @@ __device__ __forceinline__ void combine_emit(const SplitArgs& a, size_t out_row0
 }
 
 
-template <uint32_t D, bool APPEND>
+template <uint32_t D, bool APPEND, bool STREAM>
 __global__ void __launch_bounds__(256) combine_kernel(SplitArgs a) {
     const uint32_t bh = blockIdx.x;
     const uint32_t b = bh / a.g.kv_heads;
@@ -314,7 +318,7 @@ __global__ void __launch_bounds__(256) combine_kernel(SplitArgs a) {
     const size_t out_row0 = ((static_cast<size_t>(b) * a.pack + tp) * a.q_heads + static_cast<size_t>(h) * Gt +
                              (hn - tp * Gt)) * D - static_cast<size_t>(hn) * D;
     const uint32_t rec = record_floats(G, D);
-    const CombineRecords R = combine_records(a, b, h, bh, APPEND);
+    const CombineRecords<STREAM> R = combine_records<STREAM>(a, b, h, bh, rec, APPEND);
     const uint32_t slots = R.slots;
 
     constexpr uint32_t kSpec = 3;
@@ -327,7 +331,7 @@ __global__ void __launch_bounds__(256) combine_kernel(SplitArgs a) {
         ls[j] = 0.0f;
         vv[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if (sp < slots) {
-            const float* r = R.at(a, sp, rec);
+            const float* r = R.at(sp, rec);
             ms[j] = r[GD + hn];
             ls[j] = r[GD + G + hn];
             vv[j] = *reinterpret_cast<const float4*>(r + e);
@@ -344,7 +348,7 @@ __global__ void __launch_bounds__(256) combine_kernel(SplitArgs a) {
     for (uint32_t j = 0; j < kSpec; ++j)
         if (rg + 32 * j < nrec) merge_state(m, l, acc, ms[j], ls[j], vv[j]);
     for (uint32_t sp = rg + 32 * kSpec; sp < nrec; sp += 32) {
-        const float* r = R.at(a, sp, rec);
+        const float* r = R.at(sp, rec);
         merge_state(m, l, acc, r[GD + hn], r[GD + G + hn], *reinterpret_cast<const float4*>(r + e));
     }
     // Butterfly over the 8 record groups of this wave (lanes 8, 16, 32 apart).
@@ -380,7 +384,7 @@ __global__ void __launch_bounds__(256) combine_kernel(SplitArgs a) {
 // thread per 4 outputs instead of a 256-thread workgroup per 32; 8 consecutive threads
 // hold one 32-value block (Q8_1 epilogue).
 constexpr uint32_t kNarrowRecords = 8;
-template <uint32_t D, bool APPEND>
+template <uint32_t D, bool APPEND, bool STREAM>
 __global__ void __launch_bounds__(256) combine_narrow_kernel(SplitArgs a) {
     const uint32_t G = a.group;
     const uint32_t GD = G * D;
@@ -400,7 +404,7 @@ __global__ void __launch_bounds__(256) combine_narrow_kernel(SplitArgs a) {
     const size_t out_row0 = ((static_cast<size_t>(b) * a.pack + (past ? 0u : tp)) * a.q_heads +
                              static_cast<size_t>(h) * Gt + (hn - tp * Gt)) * D - static_cast<size_t>(hn) * D;
     const uint32_t rec = record_floats(G, D);
-    const CombineRecords R = combine_records(a, b, h, bhc, APPEND);
+    const CombineRecords<STREAM> R = combine_records<STREAM>(a, b, h, bhc, rec, APPEND);
     // The first batch of record slots is read before the context length arrives (slots
     // past the row set's count hold stale bytes and are dropped below; a streamed plan
     // has its count already), then the gate.
@@ -410,7 +414,7 @@ __global__ void __launch_bounds__(256) combine_narrow_kernel(SplitArgs a) {
 #pragma unroll
     for (uint32_t j = 0; j < kNarrowRecords; ++j) {
         if (j < slots) {
-            const float* r = R.at(a, j, rec);
+            const float* r = R.at(j, rec);
             ms[j] = r[GD + hn];
             ls[j] = r[GD + G + hn];
             vv[j] = *reinterpret_cast<const float4*>(r + e);
@@ -432,7 +436,7 @@ __global__ void __launch_bounds__(256) combine_narrow_kernel(SplitArgs a) {
         for (uint32_t j = 0; j < kNarrowRecords; ++j) {
             ms[j] = -INFINITY;
             if (sp0 + j < nrec) {
-                const float* r = R.at(a, sp0 + j, rec);
+                const float* r = R.at(sp0 + j, rec);
                 ms[j] = r[GD + hn];
                 ls[j] = r[GD + G + hn];
                 vv[j] = *reinterpret_cast<const float4*>(r + e);
