@@ -720,6 +720,8 @@ def test_suffix_random(gpu, seed):
 @pytest.mark.parametrize("hq,hk,d,prefix,t", [
     (32, 8, 128, 0, 1100),   # 4 waves, unsplit, odd number of row blocks paired per CU
     (24, 4, 256, 0, 1403),   # the same, even
+    (32, 16, 128, 0, 1030),  # the same, two kv heads per XCD, odd number of row blocks
+    (24, 24, 128, 0, 1300),  # the same, three
     (24, 4, 256, 0, 77),     # 4 waves, one workgroup per CU, last row block partial
     (24, 4, 256, 700, 33),   # 4 waves, split, fewer rows than two row blocks
     (32, 8, 128, 159, 129),  # 4 waves, key ranges of unequal length
