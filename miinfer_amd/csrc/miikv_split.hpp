@@ -112,9 +112,12 @@ __device__ __forceinline__ StreamTotal stream_total(const SplitArgs& a, uint32_t
     for (uint32_t off = 1; off < 64; off <<= 1) sum += __shfl_xor(sum, off, 64);
     StreamTotal t;
     t.units = sum;
-    // at least one step for each wave of a workgroup
+    // At least one step for each wave of a workgroup.  (Asking for a segment's cost on top
+    // left half the round idle in small batches: us of splits per sequence / so / now, 3
+    // sequences of 2048..4096 tokens, 32q/8kv/D128 16.6 / 17.6 / 15.9; 8 of 100..200,
+    // 24q/4kv/D256 17.2 / 21.2 / 16.9.)
     const unsigned long long q = (sum * a.g.kv_heads + a.stream_wgs - 1) / a.stream_wgs;
-    t.quota = q < kWavesPerWg + kSegmentCost ? kWavesPerWg + kSegmentCost : q;
+    t.quota = q < kWavesPerWg ? kWavesPerWg : q;
     return t;
 }
 

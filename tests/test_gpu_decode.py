@@ -453,7 +453,7 @@ def test_decode_random_batches(gpu, seed):
 
 
 @pytest.mark.parametrize("fused", [False, True])
-@pytest.mark.parametrize("hq,hk,d,f32", [(16, 4, 128, False), (24, 4, 256, True)])
+@pytest.mark.parametrize("hq,hk,d,f32", [(16, 4, 128, False), (24, 4, 256, True), (48, 4, 128, True), (48, 4, 256, True)])
 def test_decode_streamed_batch_edges(gpu, hq, hk, d, f32, fused):
     """More sequences than a wave has lanes (the streamed plan takes 64 at a time), empty
     ones, single keys, step and page edges: the runs cross sequences and kv heads at every
@@ -519,3 +519,38 @@ def test_decode_d256_steps_in_lds(gpu, mode, hq, paged, length, cap):
             s = k[h // (hq // hk)] @ q[0, h].double() / math.sqrt(d)
             expect = torch.softmax(s, 0) @ v[h // (hq // hk)]
             assert_attention_close(out[0, h].cpu().numpy(), expect.cpu().numpy(), f"{dtype} head {h}")
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("hq,hk,d,f32", [(8, 2, 128, False), (16, 8, 256, False), (48, 4, 256, True)])
+@pytest.mark.parametrize("lens", [[4000, 1, 33, 0, 2049, 128], [40, 5, 31], [1024, 4096]])
+def test_decode_streamed_small_batch(gpu, hq, hk, d, f32, lens, fused):
+    """Few sequences under a long context bound: runs of a few steps each, and with the fused
+    append the new tokens' workgroups in the same round.  Against float64 attention over the
+    dequantised cache."""
+    import miinfer_amd as m
+    rng = np.random.default_rng(sum(lens))
+    pt, stride = 256, 16
+    table = rng.permutation(len(lens) * stride).astype(np.int32).reshape(len(lens), stride)
+    cache = m.KvCache.paged_cache(hk, d, table.size, _dev(table, gpu), page_tokens=pt)
+    rows = [[_dev(randn_f16(rng, (n, hk, d)), gpu) for _ in range(2)] for n in lens]
+    new = [torch.zeros((len(lens), hk, d), dtype=torch.float16, device=gpu) for _ in range(2)]
+    for s, n in enumerate(lens):
+        stored = max(n - 1, 0) if fused else n
+        if stored:
+            cache.append(rows[s][0][:stored], rows[s][1][:stored], base_position=0, seq=s)
+        for x, r in zip(new, rows[s]):
+            if n:
+                x[s] = r[-1]
+    q = _dev(rng.standard_normal((len(lens), hq, d)).astype(np.float32), gpu)
+    q = q if f32 else q.half()
+    kw = dict(k_new=new[0], v_new=new[1]) if fused else {}
+    out, _ = m.decode_attention(cache, q, lengths=_dev(np.array(lens, np.int32), gpu), max_context=stride * pt, **kw)
+    for s, n in enumerate(lens):
+        if n == 0:
+            assert not bool(out[s].any())
+            continue
+        k, v = (x.double() for x in cache.export_dequant(s, 0, n))
+        for h in range(hq):
+            p = torch.softmax(k[h // (hq // hk)] @ q[s, h].double() / math.sqrt(d), 0)
+            assert_attention_close(out[s, h].cpu().numpy(), (p @ v[h // (hq // hk)]).cpu().numpy(), f"seq {s} head {h}")
