@@ -1333,9 +1333,8 @@ bool decode_columns_fit(uint32_t G, uint32_t D) { return G <= 16 && decode_lds_b
 // in the other 8 columns (one MFMA per block at the fp16-query register budget).
 // ragged: the last row set may be less full than the others: as few row sets as the
 // columns allow, of about equal size (7 tokens of 4 heads per kv head: 2 row sets instead
-// of 7).  Over 8000 keys, us with the store: 32q/8kv/D128 5 / 7 / 11 tokens 27.1 -> 20.0 /
-// 26.1 -> 21.2 / 39.7 -> 23.2; 24q/4kv/D256 5 / 7 / 11 26.1 -> 25.6 / 29.3 -> 26.1 / 34.6 -> 30.7.
-// (Whether a suffix runs as decodes at all is still decided by the even packing.)
+// of 7).  Whether a suffix runs as decodes at all is decided by the even packing, and which
+// packing then runs by ragged_pays.
 uint32_t suffix_pack(const miikv_view* view, uint32_t q_heads, uint32_t token_count, bool device_count,
                      uint32_t max_cols, bool ragged) {
     const uint32_t G = q_heads / view->kv_heads;
@@ -1391,6 +1390,32 @@ uint64_t suffix_by_decode_bytes_up_to(const miikv_view* view, uint32_t q_heads, 
     return most;
 }
 
+// Whether the ragged packing runs a suffix of `bound` keys faster than the even one.  Fewer,
+// fuller row sets read the keys less often, but each computes and writes more columns.
+// - An even launch of one step per wave in one resident round has nothing to save: over 300
+//   keys, 32q/8kv/D128, 7 tokens 9.0 us even, 10.0 ragged; 24q/4kv/D256 10.9 and 11.4.
+// - At two steps per wave half the row sets or fewer pay (32q/8kv/D128, 5 tokens over 2000
+//   keys 12.2 -> 10.5), three of five do not (24q/4kv/D256, 5 tokens over 4000 17.7 -> 18.2).
+// - Longer: 32q/8kv/D128, 5 / 7 / 11 tokens over 8000 21.4 -> 13.8 / 20.9 -> 15.0 / 33.6 ->
+//   16.8; 24q/4kv/D256 21.0 -> 20.6 / 24.9 -> 20.5 / 28.9 -> 24.9.
+// - An fp32 query whose even row sets hold the query's lo parts in spare columns, and whose
+//   ragged ones do not, pays for a second MFMA per block: 24q/4kv/D256, 3 tokens over 8000
+//   20.4 -> 25.0, exact 17 over 4000 30.8 -> 35.1; with a third of the row sets it is ahead
+//   (32q/8kv/D128, exact 17 over 4000 31.0 -> 18.6), and level or ahead from 33 tokens on
+//   (24q/4kv/D256, 37 over 4000 57.9 -> 56.5, 511 676 -> 548).
+static bool ragged_pays(const miikv_view* view, uint32_t q_heads, uint32_t q_dtype, uint32_t token_count, uint32_t even,
+                        uint32_t ragged, uint32_t bound) {
+    if (even == ragged) return false;
+    const uint32_t G = q_heads / view->kv_heads;
+    const uint32_t sets = (token_count + even - 1) / even, ragged_sets = (token_count + ragged - 1) / ragged;
+    if (q_dtype == MIIKV_DTYPE_F32 && 2 * G * even <= 16 && 2 * G * ragged > 16 && 3 * ragged_sets > sets && token_count <= 32)
+        return false;
+    const Plan p = make_plan(view, q_heads * even, sets, bound, kRowsetMaxCpw, true);
+    const uint64_t wgs = static_cast<uint64_t>(p.splits) * view->kv_heads * sets;
+    if (p.cpw == 1 && wgs <= kTargetWaves / kWavesPerWg) return false;
+    return p.cpw > 2 || 2 * ragged_sets <= sets;
+}
+
 miikv_status suffix_by_decode(const miikv_view* view, const void* q, uint32_t q_dtype, uint32_t q_heads, float scale,
                               uint32_t token_count, uint32_t base_position, uint32_t seq,
                               const miikv_prefill_state* prefill_state, uint32_t bound, float* out, const float* gate,
@@ -1407,9 +1432,11 @@ miikv_status suffix_by_decode(const miikv_view* view, const void* q, uint32_t q_
     // against 963 us, where twice the row sets' operand conversions cost more).
     const bool pair_cols = q_dtype == MIIKV_DTYPE_F32 && token_count >= 4 && token_count <= 16;
     const uint32_t cols = pair_cols ? kRowsetColsF32 : 16u;
-    rs.pack = suffix_pack(view, q_heads, token_count, prefill_state != nullptr, cols, true);
-    if (workspace_bytes < rowset_bytes(view, q_heads, token_count, rs.pack, bound))
-        rs.pack = suffix_pack(view, q_heads, token_count, prefill_state != nullptr, cols, false);
+    rs.pack = suffix_pack(view, q_heads, token_count, prefill_state != nullptr, cols, false);
+    const uint32_t ragged = suffix_pack(view, q_heads, token_count, prefill_state != nullptr, cols, true);
+    if (ragged_pays(view, q_heads, q_dtype, token_count, rs.pack, ragged, bound) &&
+        workspace_bytes >= rowset_bytes(view, q_heads, token_count, ragged, bound))
+        rs.pack = ragged;
     return decode_impl(view, NewRows{}, q, q_dtype, q_heads, scale, token_count, nullptr, nullptr, bound, out, gate,
                        gated_out, nullptr, workspace, workspace_bytes, stream, &rs);
 }
