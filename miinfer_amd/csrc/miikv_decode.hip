@@ -737,24 +737,31 @@ decode_kernel(SplitArgs a) {
         // bias is removed at the end with the column sums accumulated in vbias.
         if constexpr (VF16) {
             // fp16 values: P^T unscaled; keys past the context are zeroed (the memory
-            // there may hold non-finite values, and p = 0 would not cancel them)
+            // there may hold non-finite values, and p = 0 would not cancel them).  Two loops:
+            // with the choice inside, every step paid for the masks (24q/4kv/D256, 100 tokens
+            // over 4000 as decodes: 103 -> 107 us).
+            auto add_values = [&](auto masked) __attribute__((always_inline)) {
 #pragma unroll
-            for (uint32_t J = 0; J < 2; ++J) {
-                half4 pb;
+                for (uint32_t J = 0; J < 2; ++J) {
+                    half4 pb;
 #pragma unroll
-                for (uint32_t i = 0; i < 4; ++i) pb[i] = static_cast<_Float16>(s[J][i]);
+                    for (uint32_t i = 0; i < 4; ++i) pb[i] = static_cast<_Float16>(s[J][i]);
 #pragma unroll
-                for (uint32_t mt = 0; mt < NM; ++mt) {
-                    const uint4 w = v_frag(st, mt);
-                    half4 va = __builtin_bit_cast(half4, J == 0 ? make_uint2(w.x, w.y) : make_uint2(w.z, w.w));
-                    if (tail) {
+                    for (uint32_t mt = 0; mt < NM; ++mt) {
+                        const uint4 w = v_frag(st, mt);
+                        half4 va = __builtin_bit_cast(half4, J == 0 ? make_uint2(w.x, w.y) : make_uint2(w.z, w.w));
+                        if (masked) {
 #pragma unroll
-                        for (uint32_t i = 0; i < 4; ++i)
-                            if (tok0 + 16 * J + 4 * g4 + i >= Lc) va[i] = static_cast<_Float16>(0.0f);
+                            for (uint32_t i = 0; i < 4; ++i)
+                                if (tok0 + 16 * J + 4 * g4 + i >= Lc) va[i] = static_cast<_Float16>(0.0f);
+                        }
+                        O[mt] = mfma_16x16x16(va, pb, O[mt]);
                     }
-                    O[mt] = mfma_16x16x16(va, pb, O[mt]);
                 }
-            }
+            };
+            if constexpr (STREAM && D == 256) add_values(tail);  // (two loops spill registers)
+            else if (tail) add_values(std::true_type{});
+            else add_values(std::false_type{});
         } else
 #pragma unroll
         for (uint32_t J = 0; J < 2; ++J) {

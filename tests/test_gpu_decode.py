@@ -554,3 +554,35 @@ def test_decode_streamed_small_batch(gpu, hq, hk, d, f32, lens, fused):
         for h in range(hq):
             p = torch.softmax(k[h // (hq // hk)] @ q[s, h].double() / math.sqrt(d), 0)
             assert_attention_close(out[s, h].cpu().numpy(), (p @ v[h // (hq // hk)]).cpu().numpy(), f"seq {s} head {h}")
+
+
+@pytest.mark.parametrize("hq,hk,d", [(32, 8, 128), (24, 4, 256), (48, 4, 256)])
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("lens,bound", [([5000, 8192], 8192), ([4096, 1, 4000], 4096), ([33, 64, 31, 96, 100], 512),
+                                        ([64, 300, 511, 0] * 4, 2048), ([65], 512)])
+def test_decode_fp16_planes_batches(gpu, hq, hk, d, f32, lens, bound):
+    """Batches over fp16 planes, cut per sequence and streamed, with contexts that end inside a
+    step; NaN stands past every context.  Against float64 attention over the rows."""
+    import miinfer_amd as m
+    from miinfer_amd import _lib
+    rng = np.random.default_rng(sum(lens))
+    pt = 64
+    stride = bound // pt
+    table = rng.permutation(len(lens) * stride).astype(np.int32).reshape(len(lens), stride)
+    cache = m.KvCache.paged_cache(hk, d, table.size, _dev(table, gpu), page_tokens=pt, quant_mode=_lib.KV_FP16_FP16)
+    cache.k_codes.fill_(float("nan"))
+    cache.v_codes.fill_(float("nan"))
+    for s, n in enumerate(lens):
+        if n:
+            cache.append(_dev(randn_f16(rng, (n, hk, d)), gpu), _dev(randn_f16(rng, (n, hk, d)), gpu), base_position=0, seq=s)
+    q = _dev(rng.standard_normal((len(lens), hq, d)).astype(np.float32), gpu)
+    q = q if f32 else q.half()
+    out, _ = m.decode_attention(cache, q, lengths=_dev(np.array(lens, np.int32), gpu), max_context=bound)
+    for s, n in enumerate(lens):
+        if n == 0:
+            assert not bool(out[s].any())
+            continue
+        k, v = (x.double() for x in cache.export_dequant(s, 0, n))
+        for h in range(hq):
+            p = torch.softmax(k[h // (hq // hk)] @ q[s, h].double() / math.sqrt(d), 0)
+            assert_attention_close(out[s, h].cpu().numpy(), (p @ v[h // (hq // hk)]).cpu().numpy(), f"seq {s} head {h}")

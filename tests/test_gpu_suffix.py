@@ -807,3 +807,29 @@ def test_suffix_exact_at_every_accepted_workspace_size(gpu, hq, hk, d):
             expect = torch.softmax(s.masked_fill(hidden, -math.inf), -1) @ v[h // (hq // hk)]
             assert_attention_close(out[:, h].cpu().numpy(), expect.cpu().numpy(), f"{size} bytes head {h}")
     assert ran > 2
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("hq,hk,d,prefix,t", [(24, 4, 256, 2000, 17), (24, 4, 256, 2000, 37), (32, 8, 128, 2000, 17),
+                                              (32, 8, 128, 90, 37)])
+def test_suffix_exact_fp16_planes_each_packing(gpu, hq, hk, d, prefix, t, f32):
+    """Odd token counts over fp16 planes run as decodes with the even or the ragged packing,
+    an fp32 query's lo parts in spare columns or in fragments of their own, against attention
+    in float64; the memory past the context holds NaN."""
+    import miinfer_amd as m
+    from miinfer_amd import _lib
+    rng = np.random.default_rng(prefix + t)
+    n = prefix + t
+    cache = m.KvCache.contiguous(hk, d, (n + 127) // 64 * 64, quant_mode=_lib.KV_FP16_FP16)
+    for plane in (cache.k_codes, cache.v_codes):
+        plane.fill_(float("nan"))
+    cache.append(_dev(randn_f16(rng, (n, hk, d)), gpu), _dev(randn_f16(rng, (n, hk, d)), gpu))
+    q = _dev(rng.standard_normal((t, hq, d)).astype(np.float32), gpu)
+    q = q if f32 else q.half()
+    out, _ = m.suffix_attention(cache, q, prefix, exact=True)
+    k, v = (x.double() for x in cache.export_dequant(0, 0, n))
+    hidden = torch.arange(n, device=gpu)[None, :] > prefix + torch.arange(t, device=gpu)[:, None]
+    for h in range(hq):
+        s = q[:, h].double() @ k[h // (hq // hk)].T.contiguous() / math.sqrt(d)
+        expect = torch.softmax(s.masked_fill(hidden, -math.inf), -1) @ v[h // (hq // hk)]
+        assert_attention_close(out[:, h].cpu().numpy(), expect.cpu().numpy(), f"head {h}")
