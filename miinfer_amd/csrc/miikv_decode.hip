@@ -322,11 +322,14 @@ constexpr uint32_t decode_waves_per_eu() {
 // registers: K's half is refilled for the next step as soon as the scores have read it,
 // V's half after the values, so a wave always has one of them in flight (a step's codes and
 // scales take 68 registers, too many for a second set beside O and the query at two waves
-// per SIMD), and its first step is asked for before the query and the length arrive.
-// Bound: the latency of that chain, then HBM.  24q/4kv, one sequence, us a step with the
-// append, registers -> LDS: q8 200 / 4096 / 16384 / 32768 keys 10.8 -> 10.4 / 12.2 -> 11.9 /
-// 17.4 -> 16.0 / 23.4 -> 21.3 (3.3 TB/s), 9001 of at most 16384 with the K prologue 18.4 ->
-// 16.5; fp16 planes 4096 / 16384 / 32768 16.2 -> 15.8 / 24.2 -> 23.0 / 36.1 -> 32.2 (4.2 TB/s).
+// per SIMD).  The length is read ahead of the first step: with the step first, the
+// workgroups past a short context copied it all the same (200 of 32768 keys, 16q/8kv, fp16
+// planes: 15.0 us from registers, 19.5 so).
+// Bound: the latency of that chain, then HBM.  24q/4kv, one sequence, one cache again and
+// again, us with the append, registers -> LDS: q8 200 of 512 / 4096 of 4096 / 9001 of 16384 /
+// 32768 of 32768 keys 10.6 -> 10.0 / 11.7 -> 11.1 / 13.8 -> 13.1 / 21.7 -> 19.8; fp16 planes
+// 200 of 32768 / 1000 of 16384 / 9001 of 16384 / 32768 of 32768 11.0 -> 10.3 / 11.5 -> 10.7 /
+// 16.4 -> 13.7 / 30.7 -> 26.4.
 // Batches over one resident round (STREAM: 188.9 -> 199.2 at config 3) and row sets of one
 // sequence (CACHED: 25.6 -> 26.4 for 5 tokens over 8187) stay with registers.
 template <uint32_t D, bool QF32, bool APPEND, bool KF16 = false, bool VF16 = false, bool QPAIR = false,
@@ -496,18 +499,17 @@ decode_kernel(SplitArgs a) {
             }
         }
     }
+    // LDS form: the length ahead of the copies (by a scalar load, in flight with the query's
+    // loads), so that a workgroup past the sequence's splits copies nothing.
+    const uint32_t L = kLds ? split_length_scalar(a, b) : split_length(a, b);
+    // includes L == 0 (the combine kernel writes zeros)
+    if (!STREAM && split >= split_count(L, a.cpw)) return;
     if constexpr (kLds) {
-        if (n_max > 0) {
+        if (n_max > 0 && first * kChunk < L) {
             ld_slab = find_slab();
             copy_k();
             copy_v();
         }
-    }
-    const uint32_t L = kLds ? split_length_scalar(a, b) : split_length(a, b);
-    // includes L == 0 (the combine kernel writes zeros)
-    if (!STREAM && split >= split_count(L, a.cpw)) {
-        if constexpr (kLds) wait_vmem();  // the LDS must not be given up under a copy
-        return;
     }
 
     // ---- Q fragments (B operand of the QK MFMA): lane (g4, n) holds head n,
@@ -878,7 +880,9 @@ decode_kernel(SplitArgs a) {
     // waves of a workgroup then read one contiguous region at a time), otherwise each
     // wave streams its own consecutive steps.  A measured choice, not a model: config 2
     // shape, interleaved against consecutive, cpw 2 (16k) +0.3 us, cpw 4 (32k) -0.4 us,
-    // cpw 8 (64k) +0.15 us.
+    // cpw 8 (64k) +0.15 us.  The LDS form interleaves from kInterleaveCpw on: the first keys
+    // of a long capacity are then shared by the four waves (200 of 32768 keys, 16q/8kv/D256,
+    // cpw 8: 18.8 -> 11.4 us; 32768 keys 29.0 -> 28.3).
     const uint32_t rec = record_floats(G, D);
     if constexpr (STREAM) {
         // The segments of this workgroup's run (see StreamTotal).  What the loop carries is
@@ -963,7 +967,7 @@ decode_kernel(SplitArgs a) {
         // before the context length arrives from memory.
         const uint32_t cpw = a.cpw;
         const uint32_t nsteps_max = (a.max_context + kChunk - 1) / kChunk;
-        const bool interleave = cpw == kInterleaveCpw;
+        const bool interleave = kLds ? cpw >= kInterleaveCpw : cpw == kInterleaveCpw;
         const uint32_t stride = interleave ? kWavesPerWg : 1u;
         const uint32_t first = interleave ? split * kWavesPerWg * cpw + wave : (split * kWavesPerWg + wave) * cpw;
         const uint32_t last_excl = min(interleave ? (split + 1) * kWavesPerWg * cpw : first + cpw, nsteps_max);
@@ -1097,12 +1101,14 @@ constexpr uint32_t kRowsetColsF32 = MIIKV_ROWSET_COLS_F32;
 #define MIIKV_DECODE_QPAIR 1
 #endif
 namespace {
-// decode_kernel's LDS form (q8 planes, or fp16 planes from 4096 keys on: 200 / 1000 keys run
-// 13.9 / 14.6 us from registers, 14.5 / 14.9 from LDS), for launches that are neither
-// streamed nor row sets of one sequence.
+// decode_kernel's LDS form, for launches that are neither streamed nor row sets of one
+// sequence.  Over fp16 planes a workgroup takes a CU's LDS: only where each CU has at most
+// one (two of 4096..8192 keys, 24q/4kv, are 512 workgroups: 22.1 us in that form, 18.0 from
+// registers), and where a wave has a second step to fetch (24q/4kv, 1000 of 4096 keys 10.4 us
+// in LDS, 9.7 from registers).
 bool steps_in_lds(const SplitArgs& a, uint32_t D) {
     if (D != 256 || a.stream_wgs != 0 || a.rowset_order) return false;
-    return !a.g.k_f16 || a.max_context >= 4096;
+    return !a.g.k_f16 || (a.cpw > 1 && a.max_splits * a.g.kv_heads * a.batch <= 256);
 }
 template <uint32_t D, bool F32, bool APP, bool KF, bool VF>
 void launch_decode_t(dim3 grid, size_t lds, hipStream_t s, const SplitArgs& a) {

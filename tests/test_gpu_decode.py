@@ -586,3 +586,25 @@ def test_decode_fp16_planes_batches(gpu, hq, hk, d, f32, lens, bound):
         for h in range(hq):
             p = torch.softmax(k[h // (hq // hk)] @ q[s, h].double() / math.sqrt(d), 0)
             assert_attention_close(out[s, h].cpu().numpy(), (p @ v[h // (hq // hk)]).cpu().numpy(), f"seq {s} head {h}")
+
+
+@pytest.mark.parametrize("mode", ["q8", "f16"])
+@pytest.mark.parametrize("length,cap", [(1, 32768), (31, 32768), (33, 32768), (200, 32768), (1025, 16384), (32768, 32768)])
+def test_decode_d256_lds_runs_shared_by_the_waves(gpu, mode, length, cap):
+    """head_dim 256, 8 kv heads, 4 and 8 steps per wave: the waves of a workgroup take every
+    fourth step, in LDS; short contexts in a long capacity leave some waves and most
+    workgroups without keys.  Against float64 attention over the dequantised cache."""
+    import miinfer_amd as m
+    from miinfer_amd import _lib
+    hq, hk, d = 16, 8, 256
+    rng = np.random.default_rng(length)
+    cache = m.KvCache.contiguous(hk, d, cap, quant_mode=_lib.KV_Q8_Q8 if mode == "q8" else _lib.KV_FP16_FP16)
+    for t in (cache.k_codes, cache.v_codes) if mode == "f16" else (cache.k_scales, cache.v_scales):
+        t.view(torch.float16).fill_(float("nan"))  # past the context anything may stand
+    cache.append(_dev(randn_f16(rng, (length, hk, d)), gpu), _dev(randn_f16(rng, (length, hk, d)), gpu))
+    k, v = (x.double() for x in cache.export_dequant(0, 0, length))
+    q = _dev(randn_f16(rng, (1, hq, d)), gpu)
+    out, _ = m.decode_attention(cache, q, lengths=_dev(np.array([length], np.int32), gpu), max_context=cap)
+    for h in range(hq):
+        p = torch.softmax(k[h // (hq // hk)] @ q[0, h].double() / math.sqrt(d), 0)
+        assert_attention_close(out[0, h].cpu().numpy(), (p @ v[h // (hq // hk)]).cpu().numpy(), f"head {h}")
