@@ -945,7 +945,7 @@ decode_kernel(SplitArgs a) {
     } else {
         // One (sequence b, kv head h, split) of 4 waves x cpw steps per workgroup.
         uint32_t split, h, b;
-        if (a.rowset_order) {
+        if (!APPEND && !kLds && a.rowset_order) {  // (row sets are stored apart, and not in the LDS form)
             // Row sets of one sequence: items (kv head, split, row set), row sets fastest,
             // each XCD (workgroup i runs on XCD i % 8) a contiguous range of them, so the
             // workgroups an XCD runs together read the same keys (through its L2).  The
