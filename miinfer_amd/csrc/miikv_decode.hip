@@ -2,7 +2,8 @@
 //
 // Work decomposition.  A workgroup of 4 waves owns one (sequence, kv head,
 // split); a split is 4 * cpw steps of 32 tokens and each wave streams cpw
-// consecutive steps.  All G = q_heads / kv_heads query heads of the kv head are
+// steps.  In a larger batch (streamed plan, StreamTotal) it owns a run of steps
+// that may cross from one (sequence, kv head) into the next.  All G = q_heads / kv_heads query heads of the kv head are
 // served by the same wave, so every K/V byte is read from HBM exactly once.
 //
 // Per 32-token step a wave computes, for its 2 tiles of 16 tokens:
@@ -330,7 +331,7 @@ constexpr uint32_t decode_waves_per_eu() {
 // 32768 of 32768 keys 10.6 -> 10.0 / 11.7 -> 11.1 / 13.8 -> 13.1 / 21.7 -> 19.8; fp16 planes
 // 200 of 32768 / 1000 of 16384 / 9001 of 16384 / 32768 of 32768 11.0 -> 10.3 / 11.5 -> 10.7 /
 // 16.4 -> 13.7 / 30.7 -> 26.4.
-// Batches over one resident round (STREAM: 188.9 -> 199.2 at config 3) and row sets of one
+// Batches over one resident round (STREAM: 5% slower in it at config 3) and row sets of one
 // sequence (CACHED: 25.6 -> 26.4 for 5 tokens over 8187) stay with registers.
 template <uint32_t D, bool QF32, bool APPEND, bool KF16 = false, bool VF16 = false, bool QPAIR = false,
           bool CACHED = false, bool STREAM = false, bool LDS = false>
@@ -353,8 +354,9 @@ decode_kernel(SplitArgs a) {
 
     // Fused append: the last batch * kv_heads workgroups of the grid each handle the
     // new token of one (sequence, kv head).  Dispatched last, they take CU slots left
-    // free by a small grid or freed by the first split workgroups to finish, so they
-    // stay off the critical path.
+    // free by a small grid or freed by the first split workgroups to finish.  A full
+    // streamed round, whose workgroups all end together, has them after it (~4 us of 48
+    // for 48 sequences, 32q/8kv/D128); stream_workgroups leaves room for a few.
     if constexpr (APPEND) {
         const uint32_t first = gridDim.x - a.batch * a.g.kv_heads;
         if (blockIdx.x >= first) {

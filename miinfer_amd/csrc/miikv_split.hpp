@@ -34,7 +34,7 @@ struct SplitArgs {
     uint32_t max_splits;  // splits per (sequence, kv head)
     uint32_t batch;       // sequences (row-sets)
     // batch > 1, streamed plan: workgroups of the split kernel over which the batch's
-    // steps are cut evenly (stream_plan); 0: every (sequence, kv head) is cut by itself
+    // steps are cut evenly (StreamTotal); 0: every (sequence, kv head) is cut by itself
     // into splits of cpw steps per wave
     uint32_t stream_wgs;
     // [batch][kv_heads][max_splits + 1][record]: the splits, then with the fused append

@@ -1113,7 +1113,8 @@ namespace {
 // 76.3/34.2, T=16 76.8/47.0.  Without packing (a device token count), 24q/4kv/D256:
 // context 8192 T=12 41.4/36.7, T=16 42.7/46.7; context 32768 T=6 80.3/54.9, T=8
 // 80.7/77.8.  So: at most 6 row sets above a 16384-position capacity, 12 at or
-// below it.
+// below it.  (Row sets of the even packing, whichever packing then runs: a token count that
+// the columns do not divide counts its tokens one by one.)
 bool suffix_runs_as_decode(const miikv_view* v, uint32_t q_heads, uint32_t token_count, bool device_count) {
     if (!decode_columns_fit(q_heads / v->kv_heads, v->head_dim)) return false;
     if (token_count > kSuffixDecodeMaxT) return false;
@@ -1132,7 +1133,7 @@ struct SuffixPlan {
 
 // Plan for a suffix of `tokens` tokens whose keys end at or before `key_bound`:
 // the expanded tiles of every step, and enough splits to fill the chip (at least
-// 256 keys per split).  Monotone in key_bound, so a plan made with the cache
+// kSufMinKeys or kSufMinKeysSmall keys per split).  Monotone in key_bound, so a plan made with the cache
 // capacity covers any smaller context.
 // exact: the plan of suffix_exact_kernel (its tiles and its rows per workgroup).
 // waves: the form of suffix_kernel (or suffix_exact_kernel's).

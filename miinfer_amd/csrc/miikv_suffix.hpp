@@ -18,7 +18,7 @@ constexpr uint32_t kSufResidentWaves = 256 * 8;
 constexpr uint32_t kSufMaxSplits = 64;
 constexpr uint32_t kSufMinKeys = 256;  // keys per split, at least: 8-wave form
 constexpr uint32_t kSufMinKeysSmall = 160;  // 4-wave form
-// Suffixes of at most this many decode row sets (tokens / tokens packed per row set)
+// Suffixes of at most this many decode row sets (tokens / tokens per evenly packed row set)
 // run as a batch of decodes (miikv_decode.hip): caches of more than 16384 positions,
 // and of at most that many.
 constexpr uint32_t kSuffixDecodeMaxRows = 6;
@@ -63,8 +63,9 @@ struct ExpandArgs {
 // Order of (kv head, split, row block) along an XCD's workgroups: the row blocks of one
 // (kv head, split) next to each other; the splits of one row block next to each other; or,
 // without splits, each kv head's row blocks with the most keys first (kSufLongFirst), in
-// the 4-wave form the second half shortest first (kSufPaired): the two workgroups that a
-// CU then runs together have about the same keys in all.
+// the 4-wave form the second half shortest first (kSufPaired).  With whole heads on each XCD
+// (a multiple of 8 kv heads) the two workgroups that a CU then runs together have about the
+// same keys in all; with other counts some XCDs hold more long row blocks than others.
 enum SuffixOrder : uint32_t { kSufTilesTogether = 0, kSufRowsTogether = 1, kSufLongFirst = 2, kSufPaired = 3 };
 
 struct SuffixArgs {

@@ -173,9 +173,8 @@ def test_decode_rejects_bad_arguments(gpu):
 
 
 def test_decode_batch_device_chosen_split(gpu):
-    """A batch whose total context is large enough that the device raises the steps
-    per wave above the host's floor (the lengths are only known on the device): the
-    packed work items and the combine must agree on the split size."""
+    """A streamed batch of very unequal lengths (known only on the device): runs inside one
+    sequence and across several, and the combine must find every run's record."""
     import miinfer_amd as m
     rng = np.random.default_rng(31)
     hq, hk, d, pt = 32, 8, 128, 256
@@ -395,9 +394,9 @@ _WIDE_BATCHES = {10: (256, 4, 6, 16), 11: (128, 8, 4, 24), 12: (128, 8, 6, 20), 
 @pytest.mark.parametrize("seed", range(14))
 def test_decode_random_batches(gpu, seed):
     """Seeded random batches of paged decodes (batch, heads per kv head, head_dim, ragged
-    lengths including 0 and 1, context bound, query dtype, gate): the plan's split
-    size, the device's choice of steps per wave and the combine form (the wide one,
-    or one thread per 4 outputs) all vary with them; every row against the oracle."""
+    lengths including 0 and 1, context bound, query dtype, gate): the plan (cut per
+    sequence or streamed), its split size and the combine form (the wide one, or one
+    thread per 4 outputs) all vary with them; every row against the oracle."""
     import miinfer_amd as m
     rng = np.random.default_rng(1000 + seed)
     d = int(rng.choice([128, 256]))
