@@ -135,7 +135,7 @@ __global__ void __launch_bounds__(256) expand_kernel(ExpandArgs a) {
     // 4G .. +3); fragment f = 2mt + kc, lane (n, hh) holds dim 32mt + n, keys 16kc + 4hh .. +3
     // and 16kc + 8 + 4hh .. +3 (G = hh and 2 + hh).
     const uint32_t vd = tid % D, vg0 = tid / D;
-    uint2 vw[VG];
+    uint2 vw[VG] = {};  // (a step of the suffix's own keys alone reads none)
     if (!geo.v_f16 && tid < kSufStep * NB) {  // V scales to [block][key]; the suffix's own keys below
         const uint32_t key = tid / NB, blk = tid % NB;
         if (!own(key)) s_vs[blk * kSufStep + key] = tok0 + key < nkeys ? clamp_scale(vsc[tid]) : (_Float16)0.0f;
