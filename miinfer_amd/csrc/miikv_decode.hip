@@ -1407,28 +1407,41 @@ uint64_t suffix_by_decode_bytes_up_to(const miikv_view* view, uint32_t q_heads, 
 
 // Whether the ragged packing runs a suffix of `bound` keys faster than the even one.  Fewer,
 // fuller row sets read the keys less often, but each computes and writes more columns.
-// - An even launch of one step per wave in one resident round has nothing to save: over 300
-//   keys, 32q/8kv/D128, 7 tokens 9.0 us even, 10.0 ragged; 24q/4kv/D256 10.9 and 11.4.
-// - At two steps per wave half the row sets or fewer pay (32q/8kv/D128, 5 tokens over 2000
-//   keys 12.2 -> 10.5), three of five do not (24q/4kv/D256, 5 tokens over 4000 17.7 -> 18.2).
+// - One step per wave: it pays where the even launch fills more than half of the chip's waves
+//   (24q/4kv/D256, 9 tokens over 1000 keys, 1152 of 2048 waves, 15.6 -> 14.8 us; 3 over 4000,
+//   1512, 15.6 -> 13.9), not below (32q/8kv/D128, 10 over 600, 760, 9.5 -> 10.7; 7 over 300
+//   9.0 -> 10.0; 24q/4kv/D256, 3 over 2000, 756, 12.6 -> 12.8); an fp32 query's 8 columns a
+//   little earlier (32q/8kv/D128, 11 over 300, 880, 11.1 -> 9.9; 7 over 300, 560, 10.5 -> 10.9).
+// - Two steps per wave: with half the row sets or fewer (32q/8kv/D128, 5 over 2000 12.2 -> 10.5),
+//   or from 0.7 of the waves' steps on (24q/4kv/D256, 3 over 8000, 0.74, 18.1 -> 16.7; 7 over
+//   4000, 0.86, 19.0 -> 18.3), not below (11 over 2000, 0.68, 16.6 -> 17.4; 32q/8kv/D128, 10 over
+//   2000, 0.62, 13.2 -> 13.7).
 // - Longer: 32q/8kv/D128, 5 / 7 / 11 tokens over 8000 21.4 -> 13.8 / 20.9 -> 15.0 / 33.6 ->
 //   16.8; 24q/4kv/D256 21.0 -> 20.6 / 24.9 -> 20.5 / 28.9 -> 24.9.
 // - An fp32 query whose even row sets hold the query's lo parts in spare columns, and whose
-//   ragged ones do not, pays for a second MFMA per block: 24q/4kv/D256, 3 tokens over 8000
-//   20.4 -> 25.0, exact 17 over 4000 30.8 -> 35.1; with a third of the row sets it is ahead
-//   (32q/8kv/D128, exact 17 over 4000 31.0 -> 18.6), and level or ahead from 33 tokens on
-//   (24q/4kv/D256, 37 over 4000 57.9 -> 56.5, 511 676 -> 548).
+//   ragged ones do not, pays for a second MFMA per block and, at D = 256, for half of the
+//   resident workgroups: behind where those do not hold the launch (24q/4kv/D256, 3 tokens
+//   over 8000 20.4 -> 25.0, exact 17 over 4000 30.8 -> 35.1), ahead where they do (3 over 4000
+//   17.7 -> 15.9), with a third of the row sets (32q/8kv/D128, exact 17 over 4000 31.0 -> 18.6)
+//   and from 33 tokens on (24q/4kv/D256, 37 over 4000 57.9 -> 56.5, 511 676 -> 548).
 static bool ragged_pays(const miikv_view* view, uint32_t q_heads, uint32_t q_dtype, uint32_t token_count, uint32_t even,
                         uint32_t ragged, uint32_t bound) {
     if (even == ragged) return false;
     const uint32_t G = q_heads / view->kv_heads;
     const uint32_t sets = (token_count + even - 1) / even, ragged_sets = (token_count + ragged - 1) / ragged;
-    if (q_dtype == MIIKV_DTYPE_F32 && 2 * G * even <= 16 && 2 * G * ragged > 16 && 3 * ragged_sets > sets && token_count <= 32)
-        return false;
+    if (q_dtype == MIIKV_DTYPE_F32 && 2 * G * even <= 16 && 2 * G * ragged > 16 && 3 * ragged_sets > sets && token_count <= 32) {
+        const Plan r = make_plan(view, q_heads * ragged, ragged_sets, bound, kRowsetMaxCpw, true);
+        if (static_cast<uint64_t>(r.splits) * view->kv_heads * ragged_sets > resident_workgroups(view->head_dim, true, view->quant_mode))
+            return false;
+    }
     const Plan p = make_plan(view, q_heads * even, sets, bound, kRowsetMaxCpw, true);
     const uint64_t wgs = static_cast<uint64_t>(p.splits) * view->kv_heads * sets;
-    if (p.cpw == 1 && wgs <= kTargetWaves / kWavesPerWg) return false;
-    return p.cpw > 2 || 2 * ragged_sets <= sets;
+    const uint64_t steps = static_cast<uint64_t>((bound + kChunk - 1) / kChunk) * view->kv_heads * sets;
+    if (p.cpw == 1) {
+        const uint32_t part = q_dtype == MIIKV_DTYPE_F32 && 2 * G * ragged <= 16 ? 13u : 18u;  // of 32
+        return 32 * steps >= part * kTargetWaves || wgs > kTargetWaves / kWavesPerWg;
+    }
+    return p.cpw > 2 || 2 * ragged_sets <= sets || 10 * steps >= 14 * kTargetWaves;
 }
 
 miikv_status suffix_by_decode(const miikv_view* view, const void* q, uint32_t q_dtype, uint32_t q_heads, float scale,

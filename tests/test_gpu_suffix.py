@@ -748,7 +748,7 @@ def test_suffix_workgroup_forms(gpu, hq, hk, d, prefix, t):
 @pytest.mark.parametrize("hq,hk,d,prefix,t", [(32, 8, 128, 3000, 5), (32, 8, 128, 40, 7), (24, 4, 256, 2000, 11),
                                               (24, 4, 256, 61, 3), (32, 8, 128, 500, 10),
                                               (32, 8, 128, 8000, 7), (32, 8, 128, 2000, 5), (24, 4, 256, 8000, 3),
-                                              (24, 4, 256, 8000, 11)])
+                                              (24, 4, 256, 8000, 11), (24, 4, 256, 4000, 3), (32, 8, 128, 300, 11)])
 @pytest.mark.parametrize("f32", [False, True])
 def test_suffix_short_last_row_set_not_full(gpu, hq, hk, d, prefix, t, f32):
     """Token counts that the packed columns do not divide: the last row set's unused columns
