@@ -1040,12 +1040,12 @@ Plan make_plan(const miikv_view* v, uint32_t q_heads, uint32_t batch, uint32_t m
 // more than it evens out (config 3, 512 resident: 448 / 512 / 640 / 1024 workgroups
 // 192 / 191 / 224 / 199 us).  With the fused append the new tokens' workgroups follow the
 // streamed ones: where they are few they get their place in the round (6 sequences of up to
-// 2048 tokens, 48q/4kv/D256, fp32 query: 24.4 -> 22.6 us); more of them would cost the
-// streams more than their own short second round.
+// 2048 tokens, 48q/4kv/D256, fp32 query, 24 of 256: 24.4 -> 22.6 us); more of them take from
+// the streams what their short second round costs (config 3, 64 of 512, level).
 uint32_t stream_workgroups(const Plan& p, uint32_t batch, uint32_t kv_heads, uint32_t slots, bool append) {
     const uint64_t bh = static_cast<uint64_t>(batch) * kv_heads;
     if (batch == 1 || p.splits < 2 || bh * p.splits <= slots) return 0;
-    if (append && 8 * bh <= slots) slots -= static_cast<uint32_t>(bh);
+    if (append && 10 * bh <= slots) slots -= static_cast<uint32_t>(bh);
     return static_cast<uint32_t>(std::min<uint64_t>(slots, bh * (p.splits - 1)));
 }
 
